@@ -152,6 +152,17 @@ int vxa_paged_decode_workspace(int64_t n, int64_t num_heads, int64_t head_dim, i
                                int64_t split, size_t* ws_bytes);
 
 /*
+ * Workspace bytes with which vxa_paged_decode also splits the segments of a small grid (few
+ * requests) into units of 64 keys computed by workgroups of their own: the partials of every
+ * unit where that applies, otherwise the bytes of vxa_paged_decode_workspace. blk and waves as
+ * in vxa_paged_decode; max_len as in vxa_paged_decode_workspace. Either size is accepted, and
+ * both give the same bits: the smaller one computes whole segments.
+ */
+int vxa_paged_decode_units_workspace(int64_t n, int64_t num_heads, int64_t num_kv_heads,
+                                     int64_t head_dim, int64_t max_len, int64_t split, int64_t blk,
+                                     int64_t waves, size_t* ws_bytes);
+
+/*
  * Paged decode attention for one new token per request, with a fixed reduction order.
  * Replaces paged_attn.py:97-114 (`paged_decode`, device bodies `_paged_partial`
  * paged_attn.py:31-72 and `_paged_merge` paged_attn.py:75-94).

@@ -272,3 +272,39 @@ def test_random_shapes_against_the_oracle():
         b = rng.randrange(B)
         alone = _run(q[b:b + 1], kv, bt[b:b + 1], sl[b:b + 1], scale, 1, D, out_dtype, **kw)
         assert torch.equal(alone[0], o[b]), what
+
+
+@pytest.mark.parametrize("D,H,KV,BS", [(128, 8, 2, 16), (64, 8, 8, 24), (128, 16, 2, 528), (256, 4, 2, 32), (256, 8, 1, 48)])
+@pytest.mark.parametrize("split", [2048, 528, 80])
+def test_units_and_whole_segments_give_the_same_bits(monkeypatch, D, H, KV, BS, split):
+    """A small grid computes its units in workgroups of their own when the workspace holds their
+    partials, and whole segments otherwise: the same bits at every length around the edges of
+    units, slices and segments, with a device count, and NaN rows past the bound in both."""
+    L = 5000 if split > 80 else 1200
+    lens = [1, 15, 63, 64, 65, split - 1, split, split + 1, 255, 256, 257, L // 2 + 3, L - 1, L]
+    q, kv, bt, sl = make_paged(len(lens), L, BS, H, KV, D, seed=D + BS + split)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    q, kv, bt, sl = (t.cuda() for t in (q, kv, bt, sl))
+    kc, vc = kv_views(kv, D)
+    both = P._nx.paged_units_workspace
+    took = []
+
+    def run(b, units, bound, live):
+        def size(n, H, KV, D, max_len, split, blk, waves):
+            ws = both(n, H, KV, D, max_len, split, blk, waves) if units else P._nx.paged_workspace(n, H, D, max_len, split)
+            took.append(ws > P._nx.paged_workspace(n, H, D, max_len, split))
+            return ws
+
+        monkeypatch.setattr(P._nx, "paged_units_workspace", size)
+        out = torch.full((2, H, D), 7.0, device="cuda")
+        rows = slice(b, b + 2) if b + 2 <= len(lens) else slice(b - 1, b + 1)
+        n_live = torch.tensor([1], dtype=torch.int32, device="cuda") if live else None
+        P.paged_decode(q[rows], kc, vc, bt[rows], sl[rows], 0.09, out, 2, bound, split=split, n_live=n_live)
+        return out
+
+    monkeypatch.setattr(P, "MAX_LEN", L)
+    for b in range(len(lens)):
+        for bound, live in ((0, False), (L, True), (700, False)):
+            a, c = run(b, True, bound, live), run(b, False, bound, live)
+            assert torch.equal(a.view(torch.int32), c.view(torch.int32)), (lens[b], bound, live)
+    assert any(took) == (2 * KV * -(-700 // split) <= 128)  # the grids that take units

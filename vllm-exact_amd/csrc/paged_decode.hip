@@ -8,23 +8,39 @@
 // other requests, or on where the pages sit in memory.
 //
 // Kernel shape (MI355X-first, not a translation of the Triton kernel):
-//  * workgroup = (request b, KV head g, segment s); NW waves split the segment's 16-key
-//    tiles in a fixed interleave and meet in LDS through a fixed-order merge;
+//  * a segment is cut into units of 64 keys; a wave runs an online softmax over one unit at a
+//    time and merges its units (wave, wave + NW, ...) in order, the NW waves of the segment are
+//    merged in order, then the segments. A workgroup computes a whole segment of (request b, KV
+//    head g); where that leaves most CUs idle (a few requests), it computes NW units only and
+//    writes their partials, which a second kernel merges in the same order: the same bits;
 //  * S = K q^T on bf16 matrix cores (v_mfma_f32_16x16x32_bf16): rows are 16 keys of a tile,
 //    columns the G query heads of the group (bf16 x bf16 products are exact in fp32);
 //  * online softmax in base 2 on the hardware v_exp_f32, state per head kept in fp32;
 //  * P V on the vector ALU in fp32: each lane owns D/16 output dims for a quarter of the
-//    tile's keys, p arrives by ds_bpermute, V is read as 16-byte rows. fp32 p times bf16 v
-//    keeps all 24 bits of p, which is what the reference's hi/lo bf16 split of p
-//    (paged_attn.py:63-65) approximates with 2 x 8 bits on bf16 tensor cores.
+//    tile's keys, p arrives by row broadcasts (DPP), V is read as 16-byte rows. fp32 p times bf16
+//    v keeps all 24 bits of p, which is what the reference's hi/lo bf16 split of p
+//    (paged_attn.py:63-65) approximates with 2 x 8 bits on bf16 tensor cores;
 //  * K and V are read with nontemporal loads: every cache byte is read once per step, and on
 //    gfx950 a stream of permuted 8 KiB pages reads at ~6.6 TB/s that way against ~5.8 TB/s
 //    with the default cache policy (same pages, same lanes; the load policy is all that
 //    differs).
+//
+// What bounds it: HBM on large grids; on small ones the latency of a wave's tiles. A wave keeps
+// a ring of tiles in flight (32 KiB of K and V at D = 128, in registers), each refilled when its
+// tile has been used, also across units, so neither K nor V is waited for in the steady state;
+// exchanges between lane rows are lane swaps and DPP operands instead of LDS round trips; where
+// a page holds whole tiles, a row address is a scalar base and a lane offset. Measured at
+// H32/KV8/D128, page 16, event-timed calls, us, K then V read per tile with LDS
+// exchanges -> this: one request of 16384 keys 88.5 -> 22.7 (units; whole segments 35.3), of 1024
+// 44.5 -> 11.4; 4 of 16384 97.0 -> 49.7 (2.8 -> 5.4 TB/s); 32 of 1024 49.6 -> 26.1; 64 of 8192
+// 342.6 -> 339.7 (6.3 TB/s), with lengths spread over 4096..8192 298.8 -> 276.1; 256 of 1024 at
+// H16/KV2/D256, page 528: 186.5 -> 113.0. The units also shorten the fp32 sums: the error against
+// float64 fell by 18 % over 27 shapes of 64 to 16384 keys (largest 2.99e-7 -> 2.40e-7).
 // Arithmetic is compiled with -ffp-contract=off; every fused multiply-add is written
 // explicitly, so the order is the one in the source.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -49,9 +65,12 @@ struct PagedParams {
   int32_t bs_shift;  // log2(bs) when bs is a power of two, else -1
   int64_t n;
   const int32_t* n_live;  // device count of requests to compute (<= n), or null for all n
-  float* mp;  // [n][H][ns]
-  float* lp;  // [n][H][ns]
-  float* ap;  // [n][H][ns][D]
+  int32_t units;   // units of kUnit keys in a segment
+  int32_t slices;  // workgroups of a segment when its units are computed apart
+  int32_t slice_units;  // units of such a workgroup
+  float* mp;  // [n][H][ns], or [n][H][ns][units]
+  float* lp;  // as mp
+  float* ap;  // as mp, [D] each
   void* out;
   int64_t sot, soh;
   int32_t out_dtype;
@@ -69,15 +88,6 @@ __device__ inline void merge_state(float& m, float& l, float& a, float ms, float
   const float c_new = (ms == kNegInf) ? 0.0f : exp2_hw(ms - mn);
   l = fmaf(l, c_old, ls * c_new);
   a = fmaf(a, c_old, as_ * c_new);
-  m = mn;
-}
-
-// Same merge for the (m, l) pair only.
-__device__ inline void merge_ml(float& m, float& l, float ms, float ls) {
-  const float mn = fmaxf(m, ms);
-  const float c_old = (m == kNegInf) ? 0.0f : exp2_hw(m - mn);
-  const float c_new = (ms == kNegInf) ? 0.0f : exp2_hw(ms - mn);
-  l = fmaf(l, c_old, ls * c_new);
   m = mn;
 }
 
@@ -101,11 +111,99 @@ struct DimTraits {
   static constexpr int kDpl = D / 16;      // output dims per lane in P V
 };
 
-template <int D, int G, int TPG, int NW>
+// Keys of one unit: a wave's online softmax runs over one unit and its state is then merged into
+// the wave's running state, so that units can also be computed apart and merged later.
+constexpr int kUnit = 64;
+
+// Exchanges between the four 16-lane rows of a wave on the vector ALU (gfx950 lane swaps), in
+// place of ds_bpermute round trips through the LDS pipe. The fp32 pairs come back as
+// {x of the lower row or half, x of the upper}, for both sides.
+__device__ inline void swap32(float& a, float& b) {  // a's upper half <-> b's lower half
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ inline void swap16(float& a, float& b) {  // a's odd rows <-> b's even rows
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ inline float rows_max(float v) {
+  float a = v, b = v;
+  swap16(a, b);
+  v = fmaxf(a, b);
+  a = v, b = v;
+  swap32(a, b);
+  return fmaxf(a, b);
+}
+__device__ inline float rows_sum(float v) {
+  float a = v, b = v;
+  swap16(a, b);
+  v = a + b;
+  a = v, b = v;
+  swap32(a, b);
+  return a + b;
+}
+// Lane H of the caller's 16-lane row, for every lane of the row (a DPP operand, no LDS).
+template <int H>
+__device__ inline float row_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + H, 0xf, 0xf, false));
+}
+
+template <int N, typename F, int I = 0>
+__device__ inline void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, F, I + 1>(static_cast<F&&>(f));
+  }
+}
+
+// 16-byte (8-byte for D = 64) pieces of V a lane reads per key, raw.
+template <int D>
+struct VRaw {
+  static constexpr int kWords = D / 32;
+  uint32_t w[kWords];
+};
+template <int D>
+__device__ inline VRaw<D> load_v(const uint16_t* p) {
+  VRaw<D> r;
+  if constexpr (D == 64) {
+    const v2u32 u = __builtin_nontemporal_load(reinterpret_cast<const v2u32*>(p));
+    r.w[0] = u.x;
+    r.w[1] = u.y;
+  } else {
+#pragma unroll
+    for (int c = 0; c < D / 128; ++c) {
+      const v4u32 u = __builtin_nontemporal_load(reinterpret_cast<const v4u32*>(p + 8 * c));
+      r.w[4 * c] = u.x;
+      r.w[4 * c + 1] = u.y;
+      r.w[4 * c + 2] = u.z;
+      r.w[4 * c + 3] = u.w;
+    }
+  }
+  return r;
+}
+
+// Tiles of 16 keys whose K and V loads a wave has in flight when AHEAD: 128 VGPRs of them (64
+// where the accumulators of 4 or 8 heads of 256 dims need the registers: two waves a SIMD at 4).
+template <int D, int G>
+constexpr int ahead_tiles() {
+  return D == 256 ? (G >= 4 ? 1 : 2) : 4;
+}
+
+// UNITS: a workgroup computes a slice of a segment (slice_units consecutive units, the waves
+// taking them in turn) and writes each unit's partial (paged_merge_units_kernel merges them). Otherwise it computes a whole segment, each
+// wave merging its units (wave, wave + NW, ...) in order, then the waves in order. Both do the
+// same operations on the same values in the same order.
+template <int D, int G, int TPG, int NW, bool UNITS, bool AHEAD, bool ALIGNED>
 __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   static_assert(G >= 1 && G <= 16, "GQA group must fit the 16 MFMA columns");
+  static_assert(!AHEAD || TPG == 1, "loads ahead are written for one tile a step");
+  static_assert(AHEAD || !ALIGNED, "page-aligned tiles are written for loads ahead");
   constexpr int QS = DimTraits<D>::kQkSteps;
   constexpr int DPL = DimTraits<D>::kDpl;
+  constexpr int FL = G * DPL;  // accumulators of a lane
+  constexpr int QF = FL / 4;   // and the quarter of them its row owns once the rows are summed
   __shared__ float s_m[NW][G];
   __shared__ float s_l[NW][G];
   __shared__ float s_acc[NW][G][D];
@@ -116,7 +214,8 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   const int row = lane >> 4;  // S layout: key quad / PV layout: key quarter
 
   const int64_t per_seg = p.n * p.KV;
-  const int s = (int)(blockIdx.x / per_seg);
+  const int part = (int)(blockIdx.x / per_seg);  // segment, or slice of a segment
+  const int s = UNITS ? part / p.slices : part;
   const int64_t rem = blockIdx.x % per_seg;
   const int b = (int)(rem / p.KV);
   const int g = (int)(rem % p.KV);
@@ -126,18 +225,25 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   // Segments the request needs, capped at the model's NS as the fixed grid caps them. A grid
   // trimmed by the caller's bound on the batch's lengths covers every request within that
   // bound with the same segments (the same bits); a longer request gets NaN rows, written by
-  // its segment-0 workgroups, instead of a sum over fewer keys.
+  // its first workgroups, instead of a sum over fewer keys.
   const int need = min((L + p.split - 1) / p.split, p.ns_model);
   if (need > p.ns) {
-    if (s == 0)
+    if (part == 0)
       for (int idx = threadIdx.x; idx < G * D; idx += 64 * NW)
         store_f32_as(p.out, p.out_dtype, (int64_t)b * p.sot + (int64_t)(g * G + idx / D) * p.soh + idx % D,
                      __builtin_nanf(""));
     return;
   }
-  const int start = s * p.split;
-  if (start >= L) return;  // segment past the end: contributes exactly 0, never read
-  const int end = min(start + p.split, L);
+  // Keys [start, end) of this workgroup; its units start there.
+  int start = s * p.split;
+  int end = min(start + p.split, L);
+  int unit0 = 0;  // index of its first unit in the segment
+  if constexpr (UNITS) {
+    unit0 = (part % p.slices) * p.slice_units;
+    start += unit0 * kUnit;
+    end = min(end, start + p.slice_units * kUnit);
+  }
+  if (start >= end) return;  // past the end: contributes exactly 0, never read
 
   // The segment's block-table entries, staged once into LDS (dynamic shared memory sized
   // split / bs + 2 entries by the launcher).
@@ -145,9 +251,6 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   const int blk0 = page_of(p, start);
   const int npg = page_of(p, end - 1) - blk0 + 1;
   for (int i = threadIdx.x; i < npg; i += 64 * NW) s_pages[i] = p.bt[(int64_t)b * p.sbt + blk0 + i];
-  __syncthreads();
-  const int ntile = (end - start + 15) >> 4;
-  const int ngroup = (ntile + TPG - 1) / TPG;
 
   // q as the B operand: column = head (g*G + col), 8 dims per lane per MFMA step.
   v8bf qf[QS];
@@ -160,123 +263,235 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
       qf[i] = __builtin_bit_cast(v8bf, raw);
     }
   }
+  __syncthreads();
 
   const int64_t khead = (int64_t)g * p.skh;
   const int64_t vhead = (int64_t)g * p.svh;
+  auto krow_of = [&](int tile_key) {  // lane col -> key, 8 dims per lane per step
+    const int key = min(tile_key + col, end - 1);
+    return p.kc + page_offset(p, s_pages, blk0, key, p.skb, p.skp) + khead + 8 * row;
+  };
+  auto vrow_of = [&](int tile_key, int j) {
+    const int key = min(tile_key + 4 * row + j, end - 1);
+    return p.vc + page_offset(p, s_pages, blk0, key, p.svb, p.svp) + vhead + col * DPL;
+  };
+  auto load_k = [&](const uint16_t* krow, int i) {
+    return __builtin_nontemporal_load(reinterpret_cast<const v8u16*>(krow + 32 * i));
+  };
 
-  float m_run = kNegInf, l_run = 0.0f;  // per head column (S layout)
-  float acc[G][DPL];                     // PV layout: head x owned dims
+  float m_tot = kNegInf, l_tot = 0.0f;  // the wave's units so far, per head column (S layout)
+  float a_tot[QF];                       // the flat accumulators [row * QF, row * QF + QF)
 #pragma unroll
-  for (int h = 0; h < G; ++h)
-#pragma unroll
-    for (int d = 0; d < DPL; ++d) acc[h][d] = 0.0f;
+  for (int i = 0; i < QF; ++i) a_tot[i] = 0.0f;
 
-  for (int grp = wave; grp < ngroup; grp += NW) {
-    const int kbase = start + grp * 16 * TPG;
-    float sc[TPG][4];
+  // Tiles in flight per wave when AHEAD: slot (tile % PT) of the ring holds one tile's K and V.
+  constexpr int PT = AHEAD ? ahead_tiles<D, G>() : 1;
+  constexpr int kTiles = kUnit / 16;
+  static_assert(kTiles % PT == 0, "a unit's tiles walk the ring whole");
+  v8u16 kr[PT][QS];
+  VRaw<D> vr[PT][4];
+  // ALIGNED (pages of whole 16-key tiles): a tile's page comes from one LDS read per unit (lane t
+  // reads tile t's entry) and the row addresses are a scalar base and one lane offset per cache.
+  const uint32_t koff_lane = ALIGNED ? (uint32_t)((col * p.skp + 8 * row) * 2) : 0u;
+  const uint32_t voff_lane = ALIGNED ? (uint32_t)((4 * row * p.svp + col * DPL) * 2) : 0u;
+  struct TilePages {
+    int32_t page, off;  // lane t: tile t's block-table entry and its first row in the page
+  };
+  auto unit_pages = [&](int u) {  // a tile past the end takes the last key's row
+    const int key = min(start + u * kUnit + 16 * (lane & (kTiles - 1)), end - 1);
+    const int pg = page_of(p, key);
+    return TilePages{s_pages[pg - blk0], key - pg * p.bs};
+  };
+  auto issue = [&](int slot, int tile_key, const TilePages& pages, int t) {  // keys past the end repeat the last key's rows
+    if constexpr (ALIGNED) {
+      const int64_t off0 = __builtin_amdgcn_readlane(pages.off, t);
+      const int64_t page = __builtin_amdgcn_readlane(pages.page, t);
+      const char* kb = reinterpret_cast<const char*>(p.kc + page * p.skb + off0 * p.skp + khead);
+      const char* vb = reinterpret_cast<const char*>(p.vc + page * p.svb + off0 * p.svp + vhead);
+      uint32_t koff = koff_lane, voff[4];
 #pragma unroll
-    for (int t = 0; t < TPG; ++t) {
-      // K rows of this tile: lane col -> key, 8 dims per lane per step.
-      const int key = min(kbase + 16 * t + col, end - 1);
-      const uint16_t* krow = p.kc + page_offset(p, s_pages, blk0, key, p.skb, p.skp) + khead;
-      v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < 4; ++j) voff[j] = voff_lane + (uint32_t)(j * p.svp * 2);
+      const int last = max(end - 1 - tile_key, 0);  // the tile's last live key
+      if (last < 15) {
+        koff = (uint32_t)((min(col, last) * (int)p.skp + 8 * row) * 2);
 #pragma unroll
-      for (int i = 0; i < QS; ++i) {
-        const v8bf kf =
-            __builtin_bit_cast(v8bf, __builtin_nontemporal_load(reinterpret_cast<const v8u16*>(krow + 32 * i + 8 * row)));
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[i], c, 0, 0, 0);
+        for (int j = 0; j < 4; ++j) voff[j] = (uint32_t)((min(4 * row + j, last) * (int)p.svp + col * DPL) * 2);
       }
-      // c[r] = S[key kbase + 16t + 4*row + r][head col]
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kk = kbase + 16 * t + 4 * row + r;
-        sc[t][r] = (kk < end) ? c[r] * p.scale_log2 : kNegInf;
-      }
+      for (int i = 0; i < QS; ++i)
+        kr[slot][i] = __builtin_nontemporal_load(reinterpret_cast<const v8u16*>(kb + koff + 64 * i));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vr[slot][j] = load_v<D>(reinterpret_cast<const uint16_t*>(vb + voff[j]));
+    } else {
+      const uint16_t* krow = krow_of(tile_key);
+#pragma unroll
+      for (int i = 0; i < QS; ++i) kr[slot][i] = load_k(krow, i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vr[slot][j] = load_v<D>(vrow_of(tile_key, j));
     }
-    // Online softmax update for this group, fixed order.
-    float mx = kNegInf;
-#pragma unroll
-    for (int t = 0; t < TPG; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[t][r]);
-    mx = fmaxf(mx, shfl_xor_f32(mx, 16));
-    mx = fmaxf(mx, shfl_xor_f32(mx, 32));
-    const float m_new = fmaxf(m_run, mx);
-    const float alpha = exp2_hw(m_run - m_new);  // m_run == -inf -> 0
-    float psum = 0.0f;
-#pragma unroll
-    for (int t = 0; t < TPG; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        sc[t][r] = exp2_hw(sc[t][r] - m_new);
-        psum += sc[t][r];
-      }
-    psum = psum + shfl_xor_f32(psum, 16);
-    psum = psum + shfl_xor_f32(psum, 32);
-    l_run = fmaf(l_run, alpha, psum);
-    m_run = m_new;
+    asm volatile("" ::: "memory");  // issued here, ahead of the arithmetic below
+  };
+  TilePages pages = {0, 0};  // ALIGNED: of the unit whose loads are issued
 
-    // P V. Rescale the owned accumulators by each head's alpha (held by lane col == h).
+  // One unit of this wave; `next` (AHEAD): the wave has a further unit, NW units on.
+  auto unit = [&](int u, auto next) {
+    const int ubase = start + u * kUnit;
+    const int uend = min(ubase + kUnit, end);
+    float m_run = kNegInf, l_run = 0.0f;  // per head column (S layout)
+    float acc[FL];                         // PV layout: head x owned dims
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float ah = shfl_f32(alpha, h);
+    for (int i = 0; i < FL; ++i) acc[i] = 0.0f;
+
+    // One group of TPG tiles at kbase: k_at(t, i) and v_at(t, j) give its K and V.
+    auto group = [&](int kbase, auto&& k_at, auto&& v_at) {
+      float sc[TPG][4];
 #pragma unroll
-      for (int d = 0; d < DPL; ++d) acc[h][d] = acc[h][d] * ah;
-    }
+      for (int t = 0; t < TPG; ++t) {
+        v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int t = 0; t < TPG; ++t) {
+        for (int i = 0; i < QS; ++i)
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, k_at(t, i)), qf[i], c, 0, 0, 0);
+        // c[r] = S[key kbase + 16t + 4*row + r][head col]
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int key = min(kbase + 16 * t + 4 * row + j, end - 1);
-        const uint16_t* vrow = p.vc + page_offset(p, s_pages, blk0, key, p.svb, p.svp) + vhead + col * DPL;
-        float v[DPL];
-        if constexpr (DPL == 4) {
-          const v2u32 raw = __builtin_nontemporal_load(reinterpret_cast<const v2u32*>(vrow));
-          v[0] = __uint_as_float(raw.x << 16);
-          v[1] = __uint_as_float(raw.x & 0xFFFF0000u);
-          v[2] = __uint_as_float(raw.y << 16);
-          v[3] = __uint_as_float(raw.y & 0xFFFF0000u);
-        } else {
+        for (int r = 0; r < 4; ++r) {
+          const int kk = kbase + 16 * t + 4 * row + r;
+          sc[t][r] = (kk < uend) ? c[r] * p.scale_log2 : kNegInf;
+        }
+      }
+      // Online softmax update for this group, fixed order.
+      float mx = kNegInf;
 #pragma unroll
-          for (int c16 = 0; c16 < DPL / 8; ++c16) {
-            const v4u32 raw = __builtin_nontemporal_load(reinterpret_cast<const v4u32*>(vrow + 8 * c16));
-            const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+      for (int t = 0; t < TPG; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              v[8 * c16 + 2 * e] = __uint_as_float(w[e] << 16);
-              v[8 * c16 + 2 * e + 1] = __uint_as_float(w[e] & 0xFFFF0000u);
-            }
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[t][r]);
+      const float m_new = fmaxf(m_run, rows_max(mx));
+      const float alpha = exp2_hw(m_run - m_new);  // m_run == -inf -> 0
+      float psum = 0.0f;
+#pragma unroll
+      for (int t = 0; t < TPG; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sc[t][r] = exp2_hw(sc[t][r] - m_new);
+          psum += sc[t][r];
+        }
+      l_run = fmaf(l_run, alpha, rows_sum(psum));
+      m_run = m_new;
+
+      // P V. Rescale the owned accumulators by each head's alpha (held by lane col == h).
+      static_for<G>([&](auto h) {
+        const float ah = row_lane<h>(alpha);
+#pragma unroll
+        for (int d = 0; d < DPL; ++d) acc[h * DPL + d] = acc[h * DPL + d] * ah;
+      });
+#pragma unroll
+      for (int t = 0; t < TPG; ++t) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const VRaw<D> raw = v_at(t, j);
+          float v[DPL];
+#pragma unroll
+          for (int e = 0; e < DPL / 2; ++e) {
+            v[2 * e] = __uint_as_float(raw.w[e] << 16);
+            v[2 * e + 1] = __uint_as_float(raw.w[e] & 0xFFFF0000u);
           }
-        }
+          static_for<G>([&](auto h) {
+            // p for (key kbase+16t+4*row+j, head h) sits in lane (row, h), register j.
+            const float ph = row_lane<h>(sc[t][j]);
 #pragma unroll
-        for (int h = 0; h < G; ++h) {
-          // p for (key kbase+16t+4*row+j, head h) sits in lane (row, h), register j.
-          const float ph = shfl_f32(sc[t][j], (row << 4) | h);
-#pragma unroll
-          for (int d = 0; d < DPL; ++d) acc[h][d] = fmaf(ph, v[d], acc[h][d]);
+            for (int d = 0; d < DPL; ++d) acc[h * DPL + d] = fmaf(ph, v[d], acc[h * DPL + d]);
+          });
         }
       }
-    }
-  }
+    };
 
-  // Sum the four key quarters (fixed pairing, identical result in every lane).
+    if constexpr (AHEAD) {
+      TilePages following = {0, 0};
+      if constexpr (ALIGNED && decltype(next)::value) following = unit_pages(u + NW);
 #pragma unroll
-  for (int h = 0; h < G; ++h)
+      for (int t = 0; t < kTiles; ++t) {
+        if (ubase + 16 * t < uend)
+          group(ubase + 16 * t, [&](int, int i) { return kr[t % PT][i]; }, [&](int, int j) { return vr[t % PT][j]; });
+        if (t + PT < kTiles) {
+          issue(t % PT, ubase + 16 * (t + PT), pages, t + PT);
+        } else if constexpr (decltype(next)::value) {
+          if (t + PT == kTiles) pages = following;
+          issue(t % PT, ubase + NW * kUnit + 16 * (t + PT - kTiles), pages, t + PT - kTiles);
+        }
+      }
+    } else {
+      for (int kbase = ubase; kbase < uend; kbase += 16 * TPG) {
+        const uint16_t* krow[TPG];
 #pragma unroll
-    for (int d = 0; d < DPL; ++d) {
-      acc[h][d] = acc[h][d] + shfl_xor_f32(acc[h][d], 16);
-      acc[h][d] = acc[h][d] + shfl_xor_f32(acc[h][d], 32);
+        for (int t = 0; t < TPG; ++t) krow[t] = krow_of(kbase + 16 * t);
+        group(kbase, [&](int t, int i) { return load_k(krow[t], i); },
+              [&](int t, int j) { return load_v<D>(vrow_of(kbase + 16 * t, j)); });
+      }
     }
+
+    // Sum the four key quarters, each row keeping its quarter of the accumulators: rows r and
+    // r ^ 2 first, then r and r ^ 1.
+#pragma unroll
+    for (int i = 0; i < FL / 2; ++i) {
+      swap32(acc[i], acc[i + FL / 2]);
+      acc[i] = acc[i] + acc[i + FL / 2];
+    }
+#pragma unroll
+    for (int i = 0; i < QF; ++i) {
+      swap16(acc[i], acc[i + QF]);
+      acc[i] = acc[i] + acc[i + QF];
+    }
+
+    if constexpr (UNITS) {
+      const int64_t nu = (int64_t)p.ns * p.units;  // units per request and head in the workspace
+      const int64_t ui = (int64_t)s * p.units + unit0 + u;
+      if (row == 0 && col < G) {
+        const int64_t pi = ((int64_t)b * p.H + g * G + col) * nu + ui;
+        p.mp[pi] = m_run;
+        p.lp[pi] = l_run;
+      }
+#pragma unroll
+      for (int i = 0; i < QF; ++i) {
+        const int f = row * QF + i;
+        p.ap[(((int64_t)b * p.H + g * G + f / DPL) * nu + ui) * D + col * DPL + f % DPL] = acc[i];
+      }
+    } else {
+      // merge_state of the running state with the unit's, the factors computed once per head
+      const float mn = fmaxf(m_tot, m_run);
+      const float c_old = (m_tot == kNegInf) ? 0.0f : exp2_hw(m_tot - mn);
+      const float c_new = (m_run == kNegInf) ? 0.0f : exp2_hw(m_run - mn);
+      l_tot = fmaf(l_tot, c_old, l_run * c_new);
+      m_tot = mn;
+#pragma unroll
+      for (int i = 0; i < QF; ++i) {
+        const int h = (row * QF + i) / DPL;  // same for runs of DPL flats
+        a_tot[i] = fmaf(a_tot[i], shfl_f32(c_old, h), acc[i] * shfl_f32(c_new, h));
+      }
+    }
+  };
+
+  const int nunit = (end - start + kUnit - 1) / kUnit;
+  if constexpr (AHEAD) {
+    if (wave < nunit) {
+      if constexpr (ALIGNED) pages = unit_pages(wave);
+#pragma unroll
+      for (int t = 0; t < PT; ++t) issue(t, start + wave * kUnit + 16 * t, pages, t);
+      int u = wave;
+      for (; u + NW < nunit; u += NW) unit(u, std::true_type{});
+      unit(u, std::false_type{});
+    }
+  } else {
+    for (int u = wave; u < nunit; u += NW) unit(u, std::false_type{});
+  }
+  if constexpr (UNITS) return;
 
   if (row == 0 && col < G) {
-    s_m[wave][col] = m_run;
-    s_l[wave][col] = l_run;
+    s_m[wave][col] = m_tot;
+    s_l[wave][col] = l_tot;
   }
-  if (row == 0) {
 #pragma unroll
-    for (int h = 0; h < G; ++h)
-#pragma unroll
-      for (int d = 0; d < DPL; ++d) s_acc[wave][h][col * DPL + d] = acc[h][d];
+  for (int i = 0; i < QF; ++i) {
+    const int f = row * QF + i;
+    s_acc[wave][f / DPL][col * DPL + f % DPL] = a_tot[i];
   }
   __syncthreads();
 
@@ -303,6 +518,110 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
       p.ap[pi * D + d] = a;
     }
   }
+}
+
+// Merge of the units of one (request, head), one workgroup of 16 waves per (b, head), in the
+// order of the whole-segment kernel: wave w's units of a segment (w, w + NW, ...), the NW waves,
+// then the segments. A pass takes kSegs segments: their kSegs * NW unit chains go to the waves
+// (kBatch units loaded at once, so that a chain costs about one memory latency), the segments'
+// waves are merged by groups of D threads, and the first D threads append the segments.
+template <int D, int NW>
+__global__ __launch_bounds__(1024) void paged_merge_units_kernel(PagedParams p) {
+  constexpr int DPW = D / 64;
+  constexpr int kSegs = 8;
+  constexpr int kBatch = 8;
+  constexpr int kChains = kSegs * NW;
+  constexpr int kPer = kChains / 16;  // chains of a wave
+  __shared__ float c_m[kChains], c_l[kChains], c_a[kChains][D];
+  __shared__ float g_m[kSegs], g_l[kSegs], g_a[kSegs][D];
+  const int64_t bh = blockIdx.x;
+  const int b = (int)(bh / p.H);
+  const int head = (int)(bh % p.H);
+  if (p.n_live != nullptr && b >= *p.n_live) return;
+  const int L = p.sl[b];
+  const int nsb = min((L + p.split - 1) / p.split, p.ns_model);
+  if (nsb > p.ns) return;  // NaN rows, written by the partial kernel
+  if (nsb <= 0 && p.ns == 1) return;  // an empty request: as the whole-segment kernel leaves it
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t base = bh * p.ns * p.units;
+  float m = kNegInf, l = 0.0f, a = 0.0f;  // the request so far: thread d < D holds column d
+  for (int s0 = 0; s0 < nsb; s0 += kSegs) {
+    const int nseg = min(kSegs, nsb - s0);
+    // the wave's chains: c = wave + 16 q, their batches loaded together
+    float cm[kPer], cl[kPer], ca[kPer][DPW];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      cm[q] = kNegInf;
+      cl[q] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < DPW; ++j) ca[q][j] = 0.0f;
+    }
+    for (int i0 = 0; i0 * NW < p.units; i0 += kBatch) {  // units i0 .. i0 + kBatch - 1 of each chain
+      float ms[kPer][kBatch], ls[kPer][kBatch], as_[kPer][kBatch][DPW];
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) {
+        const int c = wave + 16 * q;
+        if (c >= nseg * NW) break;
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+          // a unit past the segment's last is read inside the workspace and not merged
+          const int64_t ui = base + (int64_t)(s0 + c / NW) * p.units + min((i0 + k) * NW + c % NW, p.units - 1);
+          ms[q][k] = p.mp[ui];
+          ls[q][k] = p.lp[ui];
+#pragma unroll
+          for (int j = 0; j < DPW; ++j) as_[q][k][j] = p.ap[ui * D + lane + 64 * j];
+        }
+      }
+      asm volatile("" ::: "memory");  // every load of the batch is issued before the first is used
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) {
+        const int c = wave + 16 * q;
+        if (c >= nseg * NW) break;
+        const int keys = min(p.split, L - (s0 + c / NW) * p.split);
+        const int nunit = (keys + kUnit - 1) / kUnit;  // of the segment; none past the request's end
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+          if ((i0 + k) * NW + c % NW >= nunit) break;
+          const float m0 = cm[q], l0 = cl[q];
+#pragma unroll
+          for (int j = 0; j < DPW; ++j) {
+            cm[q] = m0;
+            cl[q] = l0;
+            merge_state(cm[q], cl[q], ca[q][j], ms[q][k], ls[q][k], as_[q][k][j]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int c = wave + 16 * q;
+      if (lane == 0) {
+        c_m[c] = cm[q];
+        c_l[c] = cl[q];
+      }
+#pragma unroll
+      for (int j = 0; j < DPW; ++j) c_a[c][lane + 64 * j] = ca[q][j];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nseg * D; i += 1024) {
+      const int sg = i / D, d = i % D;
+      float sm = kNegInf, sl = 0.0f, sa = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) merge_state(sm, sl, sa, c_m[sg * NW + w], c_l[sg * NW + w], c_a[sg * NW + w][d]);
+      if (d == 0) {
+        g_m[sg] = sm;
+        g_l[sg] = sl;
+      }
+      g_a[sg][d] = sa;
+    }
+    __syncthreads();
+    if (threadIdx.x < D)
+      for (int sg = 0; sg < nseg; ++sg) merge_state(m, l, a, g_m[sg], g_l[sg], g_a[sg][threadIdx.x]);
+    // the next pass writes g_* only past its first barrier, and c_* were read before the last one
+  }
+  if (threadIdx.x < D)
+    store_f32_as(p.out, p.out_dtype, (int64_t)b * p.sot + (int64_t)head * p.soh + threadIdx.x, a / l);
 }
 
 // Fixed-order merge over the segments of one (request, head); one wave per (b, head).
@@ -366,36 +685,47 @@ __global__ __launch_bounds__(64) void paged_merge_kernel(PagedParams p) {
 // LDS bytes of a segment's block-table entries (the pages a `split`-key window can touch).
 size_t page_table_bytes(int64_t split, int64_t bs) { return (size_t)(split / bs + 2) * sizeof(int32_t); }
 
-template <int D, int G, int TPG, int NW>
+enum PagedMode { kSegments = 0, kUnits = 1 };
+
+template <int D, int G, int TPG, int NW, bool UNITS, bool AHEAD, bool ALIGNED>
 hipError_t launch_partial(const PagedParams& pp, hipStream_t st) {
-  const int64_t blocks = pp.n * pp.KV * pp.ns;
+  const int64_t blocks = pp.n * pp.KV * pp.ns * (UNITS ? pp.slices : 1);
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((paged_partial_kernel<D, G, TPG, NW>), dim3((unsigned)blocks), dim3(64 * NW),
-                     page_table_bytes(pp.split, pp.bs), st, pp);
+  const int64_t keys = UNITS ? std::min<int64_t>(pp.split, pp.slice_units * kUnit) : pp.split;
+  hipLaunchKernelGGL((paged_partial_kernel<D, G, TPG, NW, UNITS, AHEAD, ALIGNED>), dim3((unsigned)blocks), dim3(64 * NW),
+                     page_table_bytes(keys, pp.bs), st, pp);
   return hipGetLastError();
 }
 
 template <int D, int G>
-hipError_t dispatch_tpg_nw(int tpg, int nw, const PagedParams& pp, hipStream_t st) {
+hipError_t dispatch_tpg_nw(int tpg, int nw, PagedMode mode, const PagedParams& pp, hipStream_t st) {
+  // Pages of whole tiles, and lane offsets within a tile that fit 32 bits.
+  const bool aligned = pp.bs % 16 == 0 && pp.skp >= 0 && pp.svp >= 0 && pp.skp < (1 << 25) && pp.svp < (1 << 25);
   if (nw == 4) {
-    if (tpg == 1) return launch_partial<D, G, 1, 4>(pp, st);
-    if (tpg == 2) return launch_partial<D, G, 2, 4>(pp, st);
-    if (tpg == 4) return launch_partial<D, G, 4, 4>(pp, st);
+    if (tpg == 1) {
+      if (mode == kUnits)
+        return aligned ? launch_partial<D, G, 1, 4, true, true, true>(pp, st)
+                       : launch_partial<D, G, 1, 4, true, true, false>(pp, st);
+      return aligned ? launch_partial<D, G, 1, 4, false, true, true>(pp, st)
+                     : launch_partial<D, G, 1, 4, false, true, false>(pp, st);
+    }
+    if (tpg == 2) return launch_partial<D, G, 2, 4, false, false, false>(pp, st);
+    if (tpg == 4) return launch_partial<D, G, 4, 4, false, false, false>(pp, st);
   } else if (nw == 8) {
-    if (tpg == 1) return launch_partial<D, G, 1, 8>(pp, st);
-    if (tpg == 2) return launch_partial<D, G, 2, 8>(pp, st);
-    if (tpg == 4) return launch_partial<D, G, 4, 8>(pp, st);
+    if (tpg == 1) return launch_partial<D, G, 1, 8, false, false, false>(pp, st);
+    if (tpg == 2) return launch_partial<D, G, 2, 8, false, false, false>(pp, st);
+    if (tpg == 4) return launch_partial<D, G, 4, 8, false, false, false>(pp, st);
   }
   return hipErrorInvalidValue;
 }
 
 template <int D>
-hipError_t dispatch_g(int G, int tpg, int nw, const PagedParams& pp, hipStream_t st) {
+hipError_t dispatch_g(int G, int tpg, int nw, PagedMode mode, const PagedParams& pp, hipStream_t st) {
   switch (G) {
-    case 1: return dispatch_tpg_nw<D, 1>(tpg, nw, pp, st);
-    case 2: return dispatch_tpg_nw<D, 2>(tpg, nw, pp, st);
-    case 4: return dispatch_tpg_nw<D, 4>(tpg, nw, pp, st);
-    case 8: return dispatch_tpg_nw<D, 8>(tpg, nw, pp, st);
+    case 1: return dispatch_tpg_nw<D, 1>(tpg, nw, mode, pp, st);
+    case 2: return dispatch_tpg_nw<D, 2>(tpg, nw, mode, pp, st);
+    case 4: return dispatch_tpg_nw<D, 4>(tpg, nw, mode, pp, st);
+    case 8: return dispatch_tpg_nw<D, 8>(tpg, nw, mode, pp, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -405,7 +735,34 @@ int64_t num_segments(int64_t max_len, int64_t split) {
   return ns < 1 ? 1 : ns;
 }
 
+int64_t units_of(int64_t split) { return cdiv<int64_t>(split, kUnit); }
+
+// Whether the units of a grid of ns segments per request are computed apart. keys is the most
+// keys a request of the grid may have. Measured at H32/KV8/D128 (us a call, whole segments /
+// units, graph replay): 1 request of 512 keys 11.5 / 10.5, 1024 18.5 / 11.4, 16384 35.3 / 23.0
+// (64 workgroups of whole segments); 2 of 16384 (128) 43.6 / 37.0; 4 of 16384 (256) 49.7 / 61.3;
+// 16 of 1024 (128) 23.4 / 22.1; 32 of 1024 (256) 26.0 / 39.6. Past half the CUs the units'
+// partials (an eighth of the keys' bytes, written and read back) cost more than the idle CUs.
+bool use_units(int64_t n, int64_t kv_heads, int64_t ns, int64_t keys, int64_t blk, int64_t waves) {
+  return blk == 16 && waves == 4 && keys > 8 * kUnit && n * kv_heads * ns <= 128;
+}
+
+size_t units_bytes(int64_t n, int64_t num_heads, int64_t head_dim, int64_t ns, int64_t split) {
+  return (size_t)n * num_heads * ns * units_of(split) * (head_dim + 2) * sizeof(float);
+}
+
 }  // namespace
+
+extern "C" int vxa_paged_decode_units_workspace(int64_t n, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                                int64_t max_len, int64_t split, int64_t blk, int64_t waves,
+                                                size_t* ws_bytes) {
+  const int rc = vxa_paged_decode_workspace(n, num_heads, head_dim, max_len, split, ws_bytes);
+  if (rc != VXA_OK) return rc;
+  if (num_kv_heads <= 0 || blk <= 0 || waves <= 0) return VXA_ERR_ARG;
+  const int64_t ns = num_segments(max_len, split);
+  if (use_units(n, num_kv_heads, ns, max_len, blk, waves)) *ws_bytes = units_bytes(n, num_heads, head_dim, ns, split);
+  return VXA_OK;
+}
 
 extern "C" int vxa_paged_decode_workspace(int64_t n, int64_t num_heads, int64_t head_dim, int64_t max_len,
                                           int64_t split, size_t* ws_bytes) {
@@ -475,11 +832,20 @@ int paged_decode_impl(const void* q, int64_t sqt, int64_t sqh, const void* k_cac
   }
   pp.n = n;
   pp.n_live = n_live;
+  PagedMode mode = kSegments;
+  const int64_t keys = max_seq_len > 0 ? std::min(max_len, max_seq_len) : max_len;
+  if (use_units(n, num_kv_heads, ns, keys, blk, waves) && ws &&
+      ws_bytes >= units_bytes(n, num_heads, head_dim, ns, split))
+    mode = kUnits;
+  pp.units = (int32_t)units_of(split);
+  pp.slice_units = (int32_t)std::min<int64_t>(pp.units, waves);  // one unit per wave
+  pp.slices = (int32_t)cdiv<int64_t>(pp.units, pp.slice_units);
   float* wsf = reinterpret_cast<float*>(ws);
-  const int64_t nhs = n * num_heads * ns;
-  pp.mp = ns > 1 ? wsf : nullptr;
-  pp.lp = ns > 1 ? wsf + nhs : nullptr;
-  pp.ap = ns > 1 ? wsf + 2 * nhs : nullptr;
+  const int64_t nhs = n * num_heads * ns * (mode == kUnits ? pp.units : 1);
+  const bool partials = ns > 1 || mode == kUnits;
+  pp.mp = partials ? wsf : nullptr;
+  pp.lp = partials ? wsf + nhs : nullptr;
+  pp.ap = partials ? wsf + 2 * nhs : nullptr;
   pp.out = out; pp.sot = sot; pp.soh = soh; pp.out_dtype = out_dtype;
 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -487,15 +853,22 @@ int paged_decode_impl(const void* q, int64_t sqt, int64_t sqh, const void* k_cac
   const int nw = (int)waves;
   hipError_t err;
   switch (head_dim) {
-    case 64: err = dispatch_g<64>((int)G, tpg, nw, pp, st); break;
-    case 128: err = dispatch_g<128>((int)G, tpg, nw, pp, st); break;
-    default: err = dispatch_g<256>((int)G, tpg, nw, pp, st); break;
+    case 64: err = dispatch_g<64>((int)G, tpg, nw, mode, pp, st); break;
+    case 128: err = dispatch_g<128>((int)G, tpg, nw, mode, pp, st); break;
+    default: err = dispatch_g<256>((int)G, tpg, nw, mode, pp, st); break;
   }
   if (err == hipErrorInvalidValue) return VXA_ERR_UNSUPPORTED;
   if (err != hipSuccess) return VXA_ERR_LAUNCH;
-  if (ns > 1) {
-    const int64_t blocks = n * num_heads;
-    if (blocks > 0x7FFFFFFFLL) return VXA_ERR_UNSUPPORTED;
+  const int64_t blocks = n * num_heads;
+  if (partials && blocks > 0x7FFFFFFFLL) return VXA_ERR_UNSUPPORTED;
+  if (mode == kUnits) {
+    switch (head_dim) {
+      case 64: hipLaunchKernelGGL((paged_merge_units_kernel<64, 4>), dim3((unsigned)blocks), dim3(1024), 0, st, pp); break;
+      case 128: hipLaunchKernelGGL((paged_merge_units_kernel<128, 4>), dim3((unsigned)blocks), dim3(1024), 0, st, pp); break;
+      default: hipLaunchKernelGGL((paged_merge_units_kernel<256, 4>), dim3((unsigned)blocks), dim3(1024), 0, st, pp); break;
+    }
+    if (hipGetLastError() != hipSuccess) return VXA_ERR_LAUNCH;
+  } else if (ns > 1) {
     switch (head_dim) {
       case 64: hipLaunchKernelGGL(paged_merge_kernel<64>, dim3((unsigned)blocks), dim3(64), 0, st, pp); break;
       case 128: hipLaunchKernelGGL(paged_merge_kernel<128>, dim3((unsigned)blocks), dim3(64), 0, st, pp); break;

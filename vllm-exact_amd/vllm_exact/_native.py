@@ -39,6 +39,7 @@ EXPORTED = (
     "vxa_exact_linear_packed",
     "vxa_exact_linear_bf16x",
     "vxa_paged_decode_workspace",
+    "vxa_paged_decode_units_workspace",
     "vxa_paged_decode",
     "vxa_paged_decode_prefix",
     "vxa_exact_linear_op_noalloc",
@@ -72,6 +73,8 @@ _SIGNATURES = {
         [_vp, _i64, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _int, _int, ctypes.POINTER(_i32), _int, _vp],
     ),
     "vxa_paged_decode_workspace": (_int, [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_sz)]),
+    "vxa_paged_decode_units_workspace": (
+        _int, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_sz)]),
     "vxa_exact_linear_op_noalloc": (
         _int,
         [_vp, _int, _i64, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _int, _int, ctypes.POINTER(_i32), _int,
@@ -176,4 +179,12 @@ def exact_plan(M, N, K, cfg):
 def paged_workspace(n, H, D, max_len, split):
     ws = _sz()
     check(lib().vxa_paged_decode_workspace(n, H, D, max_len, split, ctypes.byref(ws)), "paged_decode_workspace")
+    return ws.value
+
+
+def paged_units_workspace(n, H, KV, D, max_len, split, blk, waves):
+    """paged_workspace, or what a small grid needs to compute its segments in units (same bits)."""
+    ws = _sz()
+    check(lib().vxa_paged_decode_units_workspace(n, H, KV, D, max_len, split, blk, waves, ctypes.byref(ws)),
+          "paged_decode_units_workspace")
     return ws.value

@@ -1,7 +1,8 @@
 """Paged decode attention with a fixed reduction order on MI355X, and the vLLM patch.
 
 Kernel (libvllm_exact_amd.so, paged_decode.hip): one workgroup per (request, KV head,
-segment of SPLIT keys). The segment length is fixed and the segment count is fixed by the
+segment of SPLIT keys), or per 256 keys of a segment when a few requests would leave the GPU
+idle (the same bits: both merge 64-key units in one order). The segment length is fixed and the segment count is fixed by the
 model's max length (paged_attn.py:3-5), so the grid is the same for every batch and the
 floating-point order of a request depends only on its own length. QK^T runs on bf16
 matrix cores (exact products, fp32 sums); the softmax is online in base 2; P V runs in fp32.
@@ -76,7 +77,7 @@ def paged_decode(query, key_cache, value_cache, block_table, seq_lens, scale, ou
     if n_live is not None and (not n_live.is_cuda or n_live.dtype != torch.int32 or n_live.numel() != 1
                                or n_live.device != query.device):
         raise ValueError("paged_decode: n_live must be a one-element int32 tensor on the query's GPU")
-    ws_bytes = _nx.paged_workspace(n, H, D, min(MAX_LEN, bound) if bound else MAX_LEN, split)
+    ws_bytes = _nx.paged_units_workspace(n, H, KV, D, min(MAX_LEN, bound) if bound else MAX_LEN, split, blk, warps)
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=query.device) if ws_bytes else None
     dev = query.device
     with torch.cuda.device(dev):
