@@ -94,6 +94,16 @@ int vxa_exact_linear(const int8_t* xh, const int8_t* xl, const int32_t* cx, cons
                      void* ws, size_t ws_bytes, vxa_stream_t stream);
 
 /*
+ * The config of a packed exact linear of [m, k] x [n, k] where no tuning table names one: the
+ * candidate with the least time in a cost model of the kernels (host arithmetic only, no device
+ * call). trunc as in vxa_exact_linear; one_launch_ok: the call may digitize inside the GEMM
+ * launch (bf16 rows, vxa_exact_linear_bf16x). Writes a cfg of 7 entries and whether it is for
+ * vxa_exact_linear_bf16x (*one_launch = 1) or vxa_exact_linear_packed (0). Speed only.
+ */
+int vxa_exact_linear_pick(int64_t m, int64_t n, int64_t k, int trunc, int one_launch_ok,
+                          int32_t* cfg, int* one_launch);
+
+/*
  * Fragment-major packed digits (the operand order of v_mfma_i32_16x16x64_i8).
  * A [rows, k] pair of digit planes (h, l) packs into cdiv(rows,16) x cdiv(k,64) blocks of
  * 2 KiB: block (rt, kt) = [h fragment | l fragment], fragment byte 16*lane + j holding

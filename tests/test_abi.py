@@ -70,6 +70,19 @@ def test_plan_rejects_bad_cfgs():
         _plan(-1, 64, 4096, (16, 64, 128, 4, 3, 8))
 
 
+def test_pick_gives_a_config_for_every_size():
+    for m in (0, 1, 4, 5, 16, 17, 64, 65, 200, 1531, 16384):
+        for n, k in ((0, 64), (1, 1), (16, 40), (5136, 2600), (151936, 4096), (64, 70000)):
+            for trunc in (True, False):
+                for ok in (True, False):
+                    cfg, one = nx.exact_pick(m, n, k, trunc, ok)
+                    sk = _plan(m, n, (k + 63) // 64 * 64, cfg)[0]
+                    assert len(cfg) == 7 and cfg[6] in (1, 2, 4)
+                    assert not one or (ok and cfg[0] == 16 and sk == 1 and m <= 64), (m, n, k, cfg)
+    with pytest.raises(ValueError):
+        nx.exact_pick(-1, 64, 64, True, True)
+
+
 def test_paged_workspace_sizes():
     # paged_attn.py:105-108: NS = max(1, cdiv(MAX_LEN, split)); partials only when NS > 1
     assert nx.paged_workspace(64, 32, 128, 1024, 1024) == 0

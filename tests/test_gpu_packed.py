@@ -101,8 +101,8 @@ XK_CFGS = tuple((bm, bn, 64 * kg, 8, 2, 8) for bm, bn, kg in K.XK_SHAPES)
 @pytest.mark.parametrize("M,N,Kd", [(256, 384, 4096), (70, 203, 1000), (130, 1000, 512), (200, 96, 640)])
 def test_xk_kernel_bitwise(F, tr, M, N, Kd):
     """The K-split kernel (K groups of waves reducing in LDS) for every instantiated tile, at 3
-    and 4 dots (shapes without a 4-dot instantiation, K splits that are not whole rounds and
-    K = 640, which has none, take the LDS-ring kernel) and split-K 1, 2, 4: fp32 output (lane
+    and 4 dots (shapes without a 4-dot instantiation take the LDS-ring kernel; K splits that are
+    not whole rounds end in a partial one) and split-K 1, 2, 4: fp32 output (lane
     stores; int64 partials when split), bf16 into a strided view (staged tile; the padding
     columns stay untouched), fp16 (staged, rows not 16-byte aligned) and F = 15 (offset terms),
     every one equal to the oracle rounded once."""
@@ -126,6 +126,41 @@ def test_xk_kernel_bitwise(F, tr, M, N, Kd):
             yh = torch.empty(M, N, device=DEV, dtype=torch.float16)
             K.exact_linear_packed(xp, wp, Kd, F, tr, out=yh, cfg=cfg)
             assert np.array_equal(yh.cpu().numpy().view(np.uint16), want_h), ("fp16", cfg)
+
+
+@pytest.mark.parametrize("Kd", [8, 64, 65, 128, 192, 250, 256, 320, 448, 512, 576, 2600])
+def test_xk_kernel_partial_round(Kd):
+    """The K-split kernel where K ends inside a round of 4 (2 K groups) or 8 (4 K groups) steps:
+    1 to 9 steps and 41, each tile at 3 dots and at 4 with offset digits (F = 15), the oracle's
+    bits."""
+    M, N = 70, 203
+    x, w = stress_xw(M, N, Kd, seed=Kd)
+    for F, tr in ((14, True), (15, False)):
+        xd, wd = K.digitize(x.to(DEV), F), K.digitize(w.to(DEV), F)
+        ref = oracle.exact_linear_c(np_digits(xd), np_digits(wd), F, tr)
+        xp, wp = K.pack_digits(xd), K.pack_digits(wd)
+        for cfg in XK_CFGS:
+            y = K.exact_linear_packed(xp, wp, Kd, F, tr, cfg=cfg + (1,))
+            assert np.array_equal(f32_bits(y.cpu().numpy()), f32_bits(ref)), (F, cfg)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,Kd", [(1, 200, 72), (5, 1040, 2600), (33, 512, 1000), (100, 336, 640), (300, 1030, 776), (700, 208, 4160)])
+def test_op_without_a_table_entry(monkeypatch, dtype, M, N, Kd):
+    """Packed op calls of shapes no table lists run the library's choice by size: the oracle's
+    bits at F = 14 and F = 15."""
+    plugin.load_table(None)
+    x, w = stress_xw(M, N, Kd, seed=M + Kd)
+    x, w = x.to(dtype), w.to(dtype)
+    rows = sorted({0, M // 2, M - 1})
+    for F, tr in ((14, True), (15, False)):
+        monkeypatch.setattr(plugin, "F", F)
+        monkeypatch.setattr(plugin, "TRUNC", tr)
+        y = torch.ops.exactmm.linear(x.to(DEV), *plugin.pack_weight(w.to(DEV)))[rows].cpu()
+        ref = oracle.exact_linear_c(oracle.digitize_c(x[rows].float().numpy(), F), oracle.digitize_c(w.float().numpy(), F), F, tr)
+        want = (oracle.bf16_rne_c(ref).reshape(len(rows), N) if dtype == torch.bfloat16
+                else ref.astype(np.float16).view(np.uint16))
+        assert np.array_equal(y.view(torch.int16).numpy().view(np.uint16), want), (F, plugin._packed_plan(M, N, Kd, dtype))
 
 
 FUSED_CFGS = tuple((16, 16 * nt, 128, nwk, c, 8, 1) for mt, nt, c, nwk in K.SMALL_SHAPES if mt == 1)

@@ -171,8 +171,7 @@ int run_exact(const ExactPlan& pl, ExactParams& ep, int trunc, bool packed, bool
     err = hipGetLastError();
   } else if (pl.family == kFamilyXw && packed && exact_xw_supported(pl.bm, pl.bn, pl.stages, pl.nwk, trunc != 0)) {
     err = launch_exact_xw(pl, ep, trunc != 0, st);
-  } else if (pl.family == kFamilyXk && packed && exact_xk_supported(pl.bm, pl.bn, pl.kg, pl.stages, pl.nwk, trunc != 0) &&
-             exact_xk_whole_rounds(pl.kg, ep.kch, ep.kpad)) {
+  } else if (pl.family == kFamilyXk && packed && exact_xk_supported(pl.bm, pl.bn, pl.kg, pl.stages, pl.nwk, trunc != 0)) {
     err = launch_exact_xk(pl, ep, trunc != 0, st);
   } else if (pl.family == kFamilyXw || pl.family == kFamilyXk || pl.family == kFamilyLds) {
     ExactPlan lp = pl;

@@ -111,5 +111,3 @@ bool exact_xw_supported(int bm, int bn, int r, int waves, bool trunc);
 // K steps split over the waves of a workgroup (exact_gemm_xk.hip), packed operands only.
 hipError_t launch_exact_xk(const ExactPlan& pl, const ExactParams& ep, bool trunc, hipStream_t st);
 bool exact_xk_supported(int bm, int bn, int kg, int r, int waves, bool trunc);
-// The K-split kernel takes K splits that are whole rounds (2 * KG steps of 64).
-bool exact_xk_whole_rounds(int kg, int64_t kch, int64_t kpad);

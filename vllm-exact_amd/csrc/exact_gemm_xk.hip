@@ -6,8 +6,9 @@
 // once, by one wave, straight into registers: a 128 x 192 tile loads 40 KiB per K step, where
 // waves split along M (each loading the whole weight column block) load 64 KiB.
 //
-// Round r covers KG * 2 K steps: K group g takes steps (r * KG + g) * 2 + {0, 1} (the launcher
-// takes only K splits of whole rounds). The x fragments of a round (KG * 2 steps x BM/16 row
+// Round r covers KG * 2 K steps: K group g takes steps (r * KG + g) * 2 + {0, 1}. A last round
+// that K ends in runs after the loop, without the loads of a next round, and each group only
+// its steps below the end. The x fragments of a round (KG * 2 steps x BM/16 row
 // tiles x 2 digit planes, 1 KiB each in MFMA lane order) go through a two-slot LDS ring filled
 // by global_load_lds_dwordx4 (gfx950 direct-to-LDS loads) split over all waves; a wave whose
 // share does not divide evenly copies some fragment twice (the same bytes to the same place).
@@ -103,7 +104,8 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
   const int64_t kb = (int64_t)split * p.kch;
   const int64_t ke = min(kb + p.kch, p.kpad);
   const int nk = (int)((ke - kb) >> 6);        // K steps of this split (kch <= 32768: at most 512)
-  const int nr = cdiv(nk, KG * kSteps);        // rounds
+  const int nr = nk / (KG * kSteps);           // whole rounds
+  const int tail = nk - nr * KG * kSteps;      // steps of the round K ends in (0: none)
   const int64_t kt0 = kb >> 6;
   const int64_t last_mt = cdiv<int64_t>(p.M, 16) - 1;
   const int64_t last_nt = cdiv<int64_t>(p.N, 16) - 1;
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
     const int8_t* lds_lane = ring + kg * kSteps * NFX * 1024 + lane * 16;
     for (int r = 0; r < nr; ++r) {
       const int slot = r & 1;
-      const int nxt = r + 1 < nr ? r + 1 : nr - 1;
+      const int nxt = tail > 0 || r + 1 < nr ? r + 1 : nr - 1;  // steps past the end are clamped
       const int8_t* stage = lds_lane + slot * kSlot;
       // x(r) landed (younger: W0(r), W1(r)); every wave is done with the slot of round r - 1
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * LW) : "memory");
@@ -233,8 +235,14 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
 #pragma unroll
       for (int f = 0; f < LW; ++f) issue_w(nxt, 1, w1, f);
     }
-    // the repeated loads past the last round still target this workgroup's LDS and registers
+    // the loads past the last round (repeats of its last step, or the round K ends in) have landed
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (tail > 0) {
+      const int8_t* stage = lds_lane + (nr & 1) * kSlot;
+      if (kg * kSteps < tail) step_mfmas(stage, w0, [](int) {});
+      if (kg * kSteps + 1 < tail) step_mfmas(stage + NFX * 1024, w1, [](int) {});
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the ring is free
+    }
   } else {
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   }
@@ -425,12 +433,6 @@ bool exact_xk_supported(int bm, int bn, int kg, int r, int waves, bool trunc) {
   VXA_XK_TABLE(VXA_XK_HAS)
 #undef VXA_XK_HAS
   return false;
-}
-
-bool exact_xk_whole_rounds(int kg, int64_t kch, int64_t kpad) {
-  const int64_t round = 64 * kSteps * (int64_t)kg;  // K extent of one round
-  const int64_t last = kpad - (cdiv<int64_t>(kpad, kch) - 1) * kch;
-  return kch % round == 0 && last % round == 0;
 }
 
 hipError_t launch_exact_xk(const ExactPlan& pl, const ExactParams& ep, bool trunc, hipStream_t st) {

@@ -32,6 +32,7 @@ EXPORTED = (
     "vxa_status_string",
     "vxa_digitize",
     "vxa_exact_linear_plan",
+    "vxa_exact_linear_pick",
     "vxa_exact_linear",
     "vxa_packed_bytes",
     "vxa_pack_digits",
@@ -55,6 +56,7 @@ _SIGNATURES = {
         [_i64, _i64, _i64, ctypes.POINTER(_i32), _int, ctypes.POINTER(_i32), ctypes.POINTER(_i64),
          ctypes.POINTER(_sz)],
     ),
+    "vxa_exact_linear_pick": (_int, [_i64, _i64, _i64, _int, _int, ctypes.POINTER(_i32), ctypes.POINTER(_int)]),
     "vxa_exact_linear": (
         _int,
         [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _int, _i64, _i64, _i64, _i64, _int, _int,
@@ -174,6 +176,14 @@ def exact_plan(M, N, K, cfg):
     check(lib().vxa_exact_linear_plan(M, N, K, arr, n, ctypes.byref(sk), ctypes.byref(kch), ctypes.byref(ws)),
           "exact_linear_plan")
     return sk.value, kch.value, ws.value
+
+
+def exact_pick(M, N, K, trunc, one_launch_ok):
+    """(cfg, one launch) of a packed exact linear call that no tuning table covers."""
+    cfg, one = (_i32 * 7)(), _int()
+    check(lib().vxa_exact_linear_pick(M, N, K, int(bool(trunc)), int(bool(one_launch_ok)), cfg, ctypes.byref(one)),
+          "exact_linear_pick")
+    return tuple(cfg), bool(one.value)
 
 
 def paged_workspace(n, H, D, max_len, split):

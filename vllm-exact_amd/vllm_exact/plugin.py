@@ -10,6 +10,7 @@ from pathlib import Path
 
 import torch
 
+from . import _native as _nx
 from . import kernels as K
 
 # set by enable()
@@ -56,7 +57,8 @@ def load_table(path):
             _N_SPLIT[key] = split
 
 
-# Built-in gfx950 configs when a shape has no table entry (speed only).
+# Built-in gfx950 configs when a shape has no table entry (speed only). Packed calls of the op
+# take the library's choice by size instead (_packed_plan).
 DEFAULT_CFGS = ((16, (16, 64, 128, 8, 1, 8, 1)), (32, (32, 64, 128, 8, 1, 8, 1)), (64, (64, 64, 128, 4, 1, 8, 1)))
 LARGE_M_CFG = (64, 64, 128, 4, 1, 8, 1)
 
@@ -102,6 +104,15 @@ def _n_split(M, N, Kd):
     return _N_SPLIT[(N, Kd)].get(next(m for m in ms if m >= M))
 
 
+def _packed_plan(M, N, Kd, dtype):
+    """(cfg, one launch) of a packed (M, N, K) call: the table's where it has the shape and a row
+    of at least M rows, otherwise the library's choice by size (exact_pick.hip; speed only). One
+    launch takes bf16 rows only."""
+    if _TABLE is not None and (N, Kd) in _TABLE and M <= max(_TABLE[(N, Kd)]):
+        return _cfg(M, N, Kd), dtype == torch.bfloat16 and _one_launch(M, N, Kd)
+    return _nx.exact_pick(M, N, Kd, TRUNC, dtype == torch.bfloat16)
+
+
 # (F, trunc, cfg, N, K[, M at F = 15]) the one-launch digitize + GEMM path refused. At F < 15
 # a refusal depends on the cfg and K (a K past 32768 columns needs a second K split); at F = 15
 # also on the grid, hence the row count. Cleared by load_table.
@@ -133,11 +144,10 @@ def exact_linear_op(x: torch.Tensor, wh: torch.Tensor, wl: torch.Tensor, cw: tor
     packed = wh.dim() == 4
     for i in range(0, M, RB):
         xb = x2[i:i + RB]
-        cfg = _cfg(xb.shape[0], N, Kd)
         if packed:
+            cfg, one_launch = _packed_plan(xb.shape[0], N, Kd, xb.dtype)
             key = _one_launch_key(cfg, xb.shape[0], N, Kd)
-            if (xb.dtype == torch.bfloat16 and _one_launch(xb.shape[0], N, Kd)
-                    and _ONE_LAUNCH_CFG.get(key, True)):
+            if one_launch and _ONE_LAUNCH_CFG.get(key, True):
                 # digitize inside the GEMM launch where the cfg allows it (same bits, one launch fewer)
                 try:
                     K.exact_linear_bf16x(xb, (wh, cw, sw), Kd, F, TRUNC, out=out[i:i + RB], cfg=cfg)
@@ -156,7 +166,8 @@ def exact_linear_op(x: torch.Tensor, wh: torch.Tensor, wl: torch.Tensor, cw: tor
                 K.exact_linear_packed(xd, (wh[:n1 // 16], cw[:n1], sw[:n1]), Kd, F, TRUNC, out=ob[:, :n1], cfg=cfg)
                 K.exact_linear_packed(xd, (wh[n1 // 16:], cw[n1:], sw[n1:]), Kd, F, TRUNC, out=ob[:, n1:], cfg=cfg2)
         else:
-            K.exact_linear(K.digitize(xb, F), (wh, wl, cw, sw), F, TRUNC, out=out[i:i + RB], cfg=cfg)
+            K.exact_linear(K.digitize(xb, F), (wh, wl, cw, sw), F, TRUNC, out=out[i:i + RB],
+                           cfg=_cfg(xb.shape[0], N, Kd))
     return out.reshape(*shp[:-1], N)
 
 
