@@ -154,6 +154,23 @@ int vxa_exact_linear_bf16x(const void* x, int64_t ldx, const int8_t* wp, const i
                            const int32_t* cfg, int cfg_len, vxa_stream_t stream);
 
 /*
+ * The exactmm::linear op on packed weights in one call: vxa_digitize_packed of x, then
+ * vxa_exact_linear_packed on the digits (the same launches and bits).
+ *   n1    0, or a multiple of 16: the GEMM then runs as two launches, columns [0, n1) with cfg and
+ *         [n1, n) with cfg2
+ *   scratch  256-byte aligned, at least the bytes of vxa_exact_linear_op_scratch with the same
+ *         sizes and cfgs: the packed digits, their sums and shifts, and the split-K partials
+ * Other arguments as vxa_digitize_packed and vxa_exact_linear_packed.
+ */
+int vxa_exact_linear_op_scratch(int64_t m, int64_t n, int64_t k, const int32_t* cfg, int cfg_len,
+                                int64_t n1, const int32_t* cfg2, int cfg2_len, size_t* bytes);
+int vxa_exact_linear_op(const void* x, int x_dtype, int64_t ldx, const int8_t* wp, const int32_t* cw,
+                        const int32_t* sw, void* out, int out_dtype, int64_t ldo, int64_t m, int64_t n,
+                        int64_t k, int f, int trunc, const int32_t* cfg, int cfg_len, int64_t n1,
+                        const int32_t* cfg2, int cfg2_len, void* scratch, size_t scratch_bytes,
+                        vxa_stream_t stream);
+
+/*
  * Workspace bytes for vxa_paged_decode: fp32 segment partials m, l [n, H, NS] and
  * acc [n, H, NS, D] with NS = max(1, cdiv(max_len, split)) (paged_attn.py:105-108).
  * Zero when NS == 1 (every request then finishes inside one segment).

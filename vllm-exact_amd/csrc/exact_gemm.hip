@@ -277,3 +277,55 @@ extern "C" int vxa_exact_linear_bf16x(const void* x, int64_t ldx, const int8_t* 
   if (err == hipErrorInvalidValue) return VXA_ERR_UNSUPPORTED;
   return err == hipSuccess ? VXA_OK : VXA_ERR_LAUNCH;
 }
+
+namespace {
+
+constexpr size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+
+// Split-K workspace of one GEMM of the op (0 columns: none).
+int op_gemm_ws(int64_t m, int64_t n, int64_t k, const int32_t* cfg, int cfg_len, size_t* ws) {
+  *ws = 0;
+  return n == 0 ? VXA_OK : vxa_exact_linear_plan(m, n, cdiv<int64_t>(k, 64) * 64, cfg, cfg_len, nullptr, nullptr, ws);
+}
+
+}  // namespace
+
+extern "C" int vxa_exact_linear_op_scratch(int64_t m, int64_t n, int64_t k, const int32_t* cfg, int cfg_len, int64_t n1,
+                                           const int32_t* cfg2, int cfg2_len, size_t* bytes) {
+  if (m < 0 || n < 0 || k < 0 || n1 < 0 || n1 > n || n1 % 16 || !bytes) return VXA_ERR_ARG;
+  size_t ws1 = 0, ws2 = 0;
+  int rc = op_gemm_ws(m, n1 ? n1 : n, k, cfg, cfg_len, &ws1);
+  if (rc == VXA_OK && n1) rc = op_gemm_ws(m, n - n1, k, cfg2, cfg2_len, &ws2);
+  if (rc != VXA_OK) return rc;
+  *bytes = align256(vxa_packed_bytes(m, k)) + 2 * align256((size_t)m * sizeof(int32_t)) + (ws1 > ws2 ? ws1 : ws2);
+  return VXA_OK;
+}
+
+extern "C" int vxa_exact_linear_op(const void* x, int x_dtype, int64_t ldx, const int8_t* wp, const int32_t* cw,
+                                   const int32_t* sw, void* out, int out_dtype, int64_t ldo, int64_t m, int64_t n,
+                                   int64_t k, int f, int trunc, const int32_t* cfg, int cfg_len, int64_t n1,
+                                   const int32_t* cfg2, int cfg2_len, void* scratch, size_t scratch_bytes,
+                                   vxa_stream_t stream) {
+  size_t need = 0;
+  int rc = vxa_exact_linear_op_scratch(m, n, k, cfg, cfg_len, n1, cfg2, cfg2_len, &need);
+  if (rc != VXA_OK) return rc;
+  if (out_dtype != VXA_F32 && out_dtype != VXA_BF16 && out_dtype != VXA_F16) return VXA_ERR_ARG;
+  if (m == 0 || n == 0) return VXA_OK;
+  if (!wp || !sw || !out || ldo < n || (uintptr_t)wp % 16 || (f == 15 && !cw)) return VXA_ERR_ARG;
+  if (!scratch || scratch_bytes < need) return VXA_ERR_WORKSPACE;
+  if ((uintptr_t)scratch % 256) return VXA_ERR_ARG;
+  int8_t* xp = static_cast<int8_t*>(scratch);
+  int32_t* cx = reinterpret_cast<int32_t*>(xp + align256(vxa_packed_bytes(m, k)));
+  int32_t* sx = cx + align256((size_t)m * sizeof(int32_t)) / sizeof(int32_t);
+  void* ws = sx + align256((size_t)m * sizeof(int32_t)) / sizeof(int32_t);
+  const size_t ws_bytes = scratch_bytes - (size_t)(static_cast<int8_t*>(ws) - xp);
+  rc = vxa_digitize_packed(x, x_dtype, m, k, ldx, xp, cx, sx, f, stream);
+  if (rc != VXA_OK) return rc;
+  rc = vxa_exact_linear_packed(xp, cx, sx, wp, cw, sw, out, out_dtype, ldo, m, n1 ? n1 : n, k, f, trunc, cfg, cfg_len,
+                               ws, ws_bytes, stream);
+  if (rc != VXA_OK || n1 == 0 || n1 == n) return rc;
+  const size_t esize = out_dtype == VXA_F32 ? 4 : 2;
+  return vxa_exact_linear_packed(xp, cx, sx, wp + vxa_packed_bytes(n1, k), cw ? cw + n1 : nullptr, sw + n1,
+                                 static_cast<int8_t*>(out) + n1 * esize, out_dtype, ldo, m, n - n1, k, f, trunc, cfg2,
+                                 cfg2_len, ws, ws_bytes, stream);
+}

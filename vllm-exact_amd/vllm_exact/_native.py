@@ -13,6 +13,7 @@ argument types, and turns status codes into Python exceptions:
 There is no fallback: if the library is missing, every GPU entry point raises.
 """
 import ctypes
+import functools
 from pathlib import Path
 
 import torch  # loads torch's HIP runtime first, so the library binds to that same runtime
@@ -44,6 +45,8 @@ EXPORTED = (
     "vxa_paged_decode",
     "vxa_paged_decode_prefix",
     "vxa_exact_linear_op_noalloc",
+    "vxa_exact_linear_op_scratch",
+    "vxa_exact_linear_op",
 )
 
 _i64, _i32, _int, _vp, _sz = ctypes.c_int64, ctypes.c_int32, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t
@@ -73,6 +76,15 @@ _SIGNATURES = {
     "vxa_exact_linear_bf16x": (
         _int,
         [_vp, _i64, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _int, _int, ctypes.POINTER(_i32), _int, _vp],
+    ),
+    "vxa_exact_linear_op_scratch": (
+        _int,
+        [_i64, _i64, _i64, ctypes.POINTER(_i32), _int, _i64, ctypes.POINTER(_i32), _int, ctypes.POINTER(_sz)],
+    ),
+    "vxa_exact_linear_op": (
+        _int,
+        [_vp, _int, _i64, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _int, _int, ctypes.POINTER(_i32), _int,
+         _i64, ctypes.POINTER(_i32), _int, _vp, _sz, _vp],
     ),
     "vxa_paged_decode_workspace": (_int, [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_sz)]),
     "vxa_paged_decode_units_workspace": (
@@ -151,6 +163,18 @@ def stream_handle(device):
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # current_stream() without the Stream object
+
+
+def launch(device, fn, *args):
+    """fn(*args, stream) with `device` current and torch's current stream on it; returns fn's status."""
+    index = device.index
+    if index == torch.cuda.current_device():
+        return fn(*args, stream_handle(device) if _raw_stream is None else _raw_stream(index))
+    with torch.cuda.device(device):
+        return fn(*args, stream_handle(device))
+
+
 def dtype_enum(dtype):
     try:
         return DTYPE_ENUM[dtype]
@@ -178,6 +202,15 @@ def exact_plan(M, N, K, cfg):
     return sk.value, kch.value, ws.value
 
 
+def op_scratch(M, N, K, cfg, n1=0, cfg2=None):
+    """(cfg array, its length, cfg2 array or None, its length, scratch bytes) of one vxa_exact_linear_op call."""
+    arr, n = cfg_array(cfg)
+    arr2, n2 = cfg_array(cfg2) if n1 else (None, 0)
+    ws = _sz()
+    check(lib().vxa_exact_linear_op_scratch(M, N, K, arr, n, n1, arr2, n2, ctypes.byref(ws)), "exact_linear_op_scratch")
+    return arr, n, arr2, n2, ws.value
+
+
 def exact_pick(M, N, K, trunc, one_launch_ok):
     """(cfg, one launch) of a packed exact linear call that no tuning table covers."""
     cfg, one = (_i32 * 7)(), _int()
@@ -192,6 +225,7 @@ def paged_workspace(n, H, D, max_len, split):
     return ws.value
 
 
+@functools.lru_cache(maxsize=1024)
 def paged_units_workspace(n, H, KV, D, max_len, split, blk, waves):
     """paged_workspace, or what a small grid needs to compute its segments in units (same bits)."""
     ws = _sz()

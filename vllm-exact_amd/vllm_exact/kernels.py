@@ -158,10 +158,8 @@ def digitize_packed(x, F, out=None):
     _check_sums("digitize_packed", cs, sh, R)
     if any(t.device != dev for t in out):
         raise ValueError("digitize_packed: outputs must be on the input's device")
-    with torch.cuda.device(dev):
-        _nx.check(_nx.lib().vxa_digitize_packed(x.data_ptr(), _nx.dtype_enum(x.dtype), R, K, x.stride(0),
-                                                packed.data_ptr(), cs.data_ptr(), sh.data_ptr(), F,
-                                                _nx.stream_handle(dev)), "digitize_packed")
+    _nx.check(_nx.launch(dev, _nx.lib().vxa_digitize_packed, x.data_ptr(), _nx.dtype_enum(x.dtype), R, K, x.stride(0),
+                         packed.data_ptr(), cs.data_ptr(), sh.data_ptr(), F), "digitize_packed")
     return out
 
 

@@ -58,7 +58,7 @@ def paged_decode(query, key_cache, value_cache, block_table, seq_lens, scale, ou
         if not t.is_cuda:
             raise ValueError("paged_decode runs the gfx950 HIP kernel and needs GPU tensors; "
                              "use paged_decode_torch for the CPU statement")
-    _nx.lib()
+    L = _nx.lib()
     if query.dtype != torch.bfloat16 or key_cache.dtype != torch.bfloat16 or value_cache.dtype != torch.bfloat16:
         raise NotImplementedError("paged_decode: query and KV cache must be bf16")
     if block_table.dtype != torch.int32 or seq_lens.dtype != torch.int32:
@@ -80,18 +80,18 @@ def paged_decode(query, key_cache, value_cache, block_table, seq_lens, scale, ou
     ws_bytes = _nx.paged_units_workspace(n, H, KV, D, min(MAX_LEN, bound) if bound else MAX_LEN, split, blk, warps)
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=query.device) if ws_bytes else None
     dev = query.device
-    with torch.cuda.device(dev):
-        st = _nx.stream_handle(dev)
-        head = (query.data_ptr(), query.stride(0), query.stride(1),
-                key_cache.data_ptr(), key_cache.stride(0), key_cache.stride(1), key_cache.stride(2),
-                value_cache.data_ptr(), value_cache.stride(0), value_cache.stride(1), value_cache.stride(2),
-                block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(), float(scale),
-                out.data_ptr(), _nx.dtype_enum(out.dtype), out.stride(0), out.stride(1), n)
-        tail = (H, KV, D, BS, int(MAX_LEN), bound, split, blk, warps, _nx.ptr(ws), ws_bytes, st)
-        if n_live is None:
-            _nx.check(_nx.lib().vxa_paged_decode(*head, *tail), "paged_decode")
-        else:
-            _nx.check(_nx.lib().vxa_paged_decode_prefix(*head, n_live.data_ptr(), *tail), "paged_decode")
+    head = (query.data_ptr(), query.stride(0), query.stride(1),
+            key_cache.data_ptr(), key_cache.stride(0), key_cache.stride(1), key_cache.stride(2),
+            value_cache.data_ptr(), value_cache.stride(0), value_cache.stride(1), value_cache.stride(2),
+            block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(), float(scale),
+            out.data_ptr(), _nx.dtype_enum(out.dtype), out.stride(0), out.stride(1), n)
+    tail = (H, KV, D, BS, int(MAX_LEN), bound, split, blk, warps, _nx.ptr(ws), ws_bytes)
+    if n_live is None:
+        status = _nx.launch(dev, L.vxa_paged_decode, *head, *tail)
+    else:
+        status = _nx.launch(dev, L.vxa_paged_decode_prefix, *head, n_live.data_ptr(), *tail)
+    if status:
+        _nx.check(status, "paged_decode")
     return out
 
 
