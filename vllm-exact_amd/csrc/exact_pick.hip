@@ -1,16 +1,21 @@
 // Which config an exact linear call of a given size runs (host code): a cost model of the
 // kernels' tiles, for shapes and row counts no tuning table covers.
 //
-// Every candidate's time is t = fixed + rounds * (round + step * K / 1024) + byte * MB, with
-// rounds = cdiv(workgroups, 256) rounds of one workgroup per CU and MB the weight digits in
-// 1e6 bytes: the rounds carry the work of a workgroup (its K steps and its fixed phases), the
-// last term the weight stream where that is longer. The coefficients (us) are least-squares fits
-// of the relative error to graph-replay timings on MI355X of each candidate at 133 (M, N, K)
-// grids x 5 (F = 14, 3 dots: 845 sizes, F = 15, 4 dots: 665), M = 1..4096, N = 512..16384, K =
-// 512..12288, weights rotated. The picked candidate then takes 1.026x (3 dots) and 1.018x
-// (4 dots) the time of the best of all 50 measured at that size on average, 1.13x and 1.10x at
-// the 95th percentile; the fixed configs by row count it replaces took 2.1x on average at M >= 96.
+// Every candidate's time is the larger of
+//   fixed + ceil(r) * (round + step * K / 1024) + byte * MB   and   r * (many_round + many_step * K / 1024)
+// with r = workgroups / 256, the rounds of one workgroup per CU, and MB the weight digits in 1e6
+// bytes. A round carries the work of a workgroup (its fixed phases and its K steps), MB the weight
+// stream where that is longer. Over many rounds a partly filled last one counts by its share, and a
+// round takes longer: these kernels are power-bound and the chip then holds a lower clock. The
+// coefficients (us) are least-squares fits of the relative error to graph-replay timings on MI355X
+// of each candidate at 979 sizes (F = 14, 3 dots) and 749 (F = 15, 4 dots), M = 1..8192, N =
+// 512..24576, K = 512..12288, weights rotated. Digitize and GEMM of the picked candidate take
+// 1.023x (3 dots) and 1.017x (4 dots) the time of the best of all configs measured at that size on
+// average, 1.11x and 1.10x at the 95th percentile (1.009x and 1.006x on average from 1024 rows
+// up); the fixed configs by row count that it replaces took 1.8x below 96 rows and 1.9x from there
+// to 1024. 1531 rows of fp16 through 5136 x 2600: 163.6 -> 66 us.
 
+#include <algorithm>
 #include <cmath>
 
 #include "exact_gemm_common.h"
@@ -23,70 +28,72 @@ struct Candidate {
   bool one_launch;   // digitize inside the GEMM launch
   int64_t max_rows;  // taken up to this many rows
   int32_t bm, bn, bk, waves, stages;
-  float fixed, round, step, byte;
+  float fixed, round, step, byte, many_round, many_step;
 };
 
 constexpr Candidate kThreeDots[] = {
-    {false, kAnyRows, 16, 16, 128, 8, 1, 2.613f, 0.168f, 0.647f, 0.079f},
-    {false, kAnyRows, 16, 16, 128, 16, 1, 2.163f, 0.626f, 0.580f, 0.085f},
-    {false, kAnyRows, 16, 32, 128, 4, 1, 3.180f, 0.000f, 0.995f, 0.096f},
-    {false, kAnyRows, 16, 32, 128, 8, 1, 2.473f, 0.495f, 0.713f, 0.109f},
-    {false, kAnyRows, 32, 16, 128, 8, 1, 2.557f, 0.264f, 0.924f, 0.068f},
-    {false, kAnyRows, 32, 32, 128, 4, 1, 3.513f, 0.269f, 1.348f, 0.083f},
-    {false, kAnyRows, 32, 32, 128, 8, 1, 2.829f, 0.534f, 1.335f, 0.088f},
-    {false, kAnyRows, 32, 128, 64, 4, 4, 4.248f, 0.686f, 3.728f, 0.070f},
-    {false, kAnyRows, 64, 16, 128, 8, 1, 2.600f, 0.880f, 1.651f, 0.062f},
-    {false, kAnyRows, 64, 32, 128, 8, 1, 3.098f, 1.498f, 1.979f, 0.082f},
-    {false, kAnyRows, 64, 64, 256, 8, 2, 0.620f, 4.043f, 2.847f, 0.082f},
-    {false, kAnyRows, 64, 96, 256, 8, 2, 0.720f, 5.185f, 3.511f, 0.091f},
-    {false, kAnyRows, 64, 128, 128, 8, 2, 2.362f, 2.235f, 4.255f, 0.100f},
-    {false, kAnyRows, 64, 192, 128, 8, 2, 0.160f, 5.749f, 5.710f, 0.121f},
-    {false, kAnyRows, 128, 128, 128, 8, 2, 0.000f, 7.254f, 6.593f, 0.077f},
-    {false, kAnyRows, 128, 192, 128, 8, 2, 0.000f, 9.454f, 9.756f, 0.044f},
-    {true, 4, 16, 16, 128, 8, 1, 3.162f, 0.460f, 1.367f, 0.000f},
-    {true, 64, 16, 16, 128, 8, 1, 2.742f, 0.532f, 1.882f, 0.000f},
-    {true, 4, 16, 16, 128, 16, 1, 2.584f, 1.550f, 0.939f, 0.034f},
-    {true, 64, 16, 16, 128, 16, 1, 2.480f, 1.242f, 1.584f, 0.000f},
-    {true, 4, 16, 32, 128, 8, 1, 2.365f, 1.263f, 1.515f, 0.060f},
-    {true, 64, 16, 32, 128, 8, 1, 2.253f, 1.041f, 2.180f, 0.047f},
-    {true, 4, 16, 32, 128, 16, 1, 0.000f, 3.970f, 1.381f, 0.065f},
-    {true, 64, 16, 32, 128, 16, 1, 0.936f, 2.753f, 1.987f, 0.052f},
-    {true, 4, 16, 64, 128, 8, 1, 0.000f, 3.714f, 2.001f, 0.095f},
-    {true, 64, 16, 64, 128, 8, 1, 1.487f, 2.136f, 2.986f, 0.079f},
+    {false, kAnyRows, 16, 16, 128, 8, 1, 2.552f, 0.184f, 0.665f, 0.078f, 0.000f, 0.000f},
+    {false, kAnyRows, 16, 16, 128, 16, 1, 2.087f, 0.653f, 0.600f, 0.084f, 0.000f, 0.000f},
+    {false, kAnyRows, 16, 32, 128, 4, 1, 3.172f, 0.000f, 0.993f, 0.097f, 0.000f, 0.000f},
+    {false, kAnyRows, 16, 32, 128, 8, 1, 2.357f, 0.560f, 0.727f, 0.110f, 0.000f, 0.000f},
+    {false, kAnyRows, 32, 16, 128, 8, 1, 2.501f, 0.263f, 0.937f, 0.072f, 0.000f, 0.000f},
+    {false, kAnyRows, 32, 32, 128, 4, 1, 3.454f, 0.278f, 1.363f, 0.083f, 0.000f, 0.000f},
+    {false, kAnyRows, 32, 32, 128, 8, 1, 2.770f, 0.547f, 1.349f, 0.090f, 0.000f, 0.000f},
+    {false, kAnyRows, 32, 128, 64, 4, 4, 4.235f, 0.700f, 3.702f, 0.075f, 0.000f, 0.000f},
+    {false, kAnyRows, 64, 16, 128, 8, 1, 2.574f, 0.885f, 1.635f, 0.071f, 0.000f, 0.000f},
+    {false, kAnyRows, 64, 32, 128, 8, 1, 3.070f, 1.508f, 1.964f, 0.088f, 0.000f, 0.000f},
+    {false, kAnyRows, 64, 64, 256, 8, 2, 1.380f, 3.691f, 2.462f, 0.105f, 3.125f, 4.133f},
+    {false, kAnyRows, 64, 96, 256, 8, 2, 1.597f, 4.612f, 3.265f, 0.105f, 4.820f, 5.091f},
+    {false, kAnyRows, 64, 128, 128, 8, 2, 2.814f, 1.997f, 4.068f, 0.106f, 2.032f, 5.394f},
+    {false, kAnyRows, 64, 192, 128, 8, 2, 0.893f, 5.164f, 5.574f, 0.126f, 5.558f, 7.819f},
+    {false, kAnyRows, 128, 128, 128, 8, 2, 0.000f, 7.203f, 6.340f, 0.076f, 6.508f, 9.486f},
+    {false, kAnyRows, 128, 192, 128, 8, 2, 0.000f, 9.423f, 9.631f, 0.046f, 10.047f, 13.239f},
+    {true, 4, 16, 16, 128, 8, 1, 3.162f, 0.460f, 1.367f, 0.000f, 0.000f, 0.000f},
+    {true, 64, 16, 16, 128, 8, 1, 2.764f, 0.527f, 1.874f, 0.000f, 0.000f, 0.000f},
+    {true, 4, 16, 16, 128, 16, 1, 2.584f, 1.550f, 0.939f, 0.034f, 0.000f, 0.000f},
+    {true, 64, 16, 16, 128, 16, 1, 2.447f, 1.253f, 1.593f, 0.000f, 0.000f, 0.000f},
+    {true, 4, 16, 32, 128, 8, 1, 2.365f, 1.263f, 1.515f, 0.060f, 0.000f, 0.000f},
+    {true, 64, 16, 32, 128, 8, 1, 2.231f, 1.054f, 2.186f, 0.046f, 0.000f, 0.000f},
+    {true, 4, 16, 32, 128, 16, 1, 0.000f, 3.970f, 1.381f, 0.065f, 0.000f, 0.000f},
+    {true, 64, 16, 32, 128, 16, 1, 0.833f, 2.820f, 2.003f, 0.052f, 0.000f, 0.000f},
+    {true, 4, 16, 64, 128, 8, 1, 0.000f, 3.714f, 2.001f, 0.095f, 0.000f, 0.000f},
+    {true, 64, 16, 64, 128, 8, 1, 1.345f, 2.256f, 2.989f, 0.080f, 0.000f, 0.000f},
 };
 
 constexpr Candidate kFourDots[] = {
-    {false, kAnyRows, 16, 16, 128, 8, 1, 2.696f, 0.185f, 0.681f, 0.076f},
-    {false, kAnyRows, 16, 16, 128, 16, 1, 2.250f, 0.692f, 0.623f, 0.076f},
-    {false, kAnyRows, 16, 32, 128, 4, 1, 3.320f, 0.017f, 1.017f, 0.101f},
-    {false, kAnyRows, 16, 32, 128, 8, 1, 2.796f, 0.331f, 0.989f, 0.107f},
-    {false, kAnyRows, 32, 16, 128, 8, 1, 2.748f, 0.424f, 0.984f, 0.076f},
-    {false, kAnyRows, 32, 32, 128, 4, 1, 3.677f, 0.593f, 1.410f, 0.080f},
-    {false, kAnyRows, 32, 32, 128, 8, 1, 2.565f, 1.044f, 1.381f, 0.086f},
-    {false, kAnyRows, 32, 128, 64, 4, 4, 6.230f, 1.777f, 4.229f, 0.052f},
-    {false, kAnyRows, 64, 16, 128, 8, 1, 2.682f, 1.097f, 1.656f, 0.051f},
-    {false, kAnyRows, 64, 32, 128, 8, 1, 0.356f, 4.160f, 2.531f, 0.090f},
-    {false, kAnyRows, 64, 64, 256, 8, 2, 0.642f, 6.476f, 3.169f, 0.071f},
-    {false, kAnyRows, 64, 96, 256, 8, 2, 0.703f, 8.977f, 3.897f, 0.073f},
-    {false, kAnyRows, 64, 128, 128, 8, 2, 0.000f, 8.989f, 5.086f, 0.072f},
-    {false, kAnyRows, 64, 192, 128, 8, 2, 0.000f, 12.544f, 6.816f, 0.086f},
-    {false, kAnyRows, 128, 128, 128, 8, 2, 0.000f, 16.151f, 8.685f, 0.042f},
-    {true, 4, 16, 16, 128, 8, 1, 3.047f, 0.801f, 1.440f, 0.000f},
-    {true, 64, 16, 16, 128, 8, 1, 2.635f, 0.992f, 1.898f, 0.000f},
-    {true, 4, 16, 16, 128, 16, 1, 2.414f, 2.021f, 1.209f, 0.007f},
-    {true, 64, 16, 16, 128, 16, 1, 1.762f, 2.505f, 1.660f, 0.000f},
-    {true, 4, 16, 32, 128, 8, 1, 2.816f, 1.105f, 1.504f, 0.066f},
-    {true, 64, 16, 32, 128, 8, 1, 2.154f, 1.603f, 2.127f, 0.048f},
-    {true, 4, 16, 32, 128, 16, 1, 1.483f, 3.549f, 1.327f, 0.075f},
-    {true, 64, 16, 32, 128, 16, 1, 1.175f, 3.178f, 2.134f, 0.046f},
-    {true, 4, 16, 64, 128, 8, 1, 0.000f, 4.249f, 1.990f, 0.092f},
-    {true, 64, 16, 64, 128, 8, 1, 0.000f, 4.341f, 2.965f, 0.084f},
+    {false, kAnyRows, 16, 16, 128, 8, 1, 2.696f, 0.185f, 0.681f, 0.076f, 0.000f, 0.000f},
+    {false, kAnyRows, 16, 16, 128, 16, 1, 2.250f, 0.692f, 0.623f, 0.076f, 0.000f, 0.000f},
+    {false, kAnyRows, 16, 32, 128, 4, 1, 3.320f, 0.017f, 1.017f, 0.101f, 0.000f, 0.000f},
+    {false, kAnyRows, 16, 32, 128, 8, 1, 2.796f, 0.331f, 0.989f, 0.107f, 0.000f, 0.000f},
+    {false, kAnyRows, 32, 16, 128, 8, 1, 2.748f, 0.424f, 0.984f, 0.076f, 0.000f, 0.000f},
+    {false, kAnyRows, 32, 32, 128, 4, 1, 3.677f, 0.593f, 1.410f, 0.080f, 0.000f, 0.000f},
+    {false, kAnyRows, 32, 32, 128, 8, 1, 2.565f, 1.044f, 1.381f, 0.086f, 0.000f, 0.000f},
+    {false, kAnyRows, 32, 128, 64, 4, 4, 6.186f, 1.870f, 4.159f, 0.056f, 0.000f, 0.000f},
+    {false, kAnyRows, 64, 16, 128, 8, 1, 2.682f, 1.097f, 1.656f, 0.051f, 0.000f, 0.000f},
+    {false, kAnyRows, 64, 32, 128, 8, 1, 0.356f, 4.160f, 2.531f, 0.090f, 0.000f, 0.000f},
+    {false, kAnyRows, 64, 64, 256, 8, 2, 1.475f, 6.174f, 2.634f, 0.098f, 5.679f, 4.238f},
+    {false, kAnyRows, 64, 96, 256, 8, 2, 1.536f, 8.496f, 3.598f, 0.088f, 8.938f, 5.258f},
+    {false, kAnyRows, 64, 128, 128, 8, 2, 0.499f, 8.739f, 4.730f, 0.085f, 8.142f, 6.367f},
+    {false, kAnyRows, 64, 192, 128, 8, 2, 0.514f, 12.199f, 6.618f, 0.093f, 12.964f, 8.679f},
+    {false, kAnyRows, 128, 128, 128, 8, 2, 0.000f, 16.201f, 8.395f, 0.029f, 15.379f, 11.051f},
+    {true, 4, 16, 16, 128, 8, 1, 3.047f, 0.801f, 1.440f, 0.000f, 0.000f, 0.000f},
+    {true, 64, 16, 16, 128, 8, 1, 2.635f, 0.992f, 1.898f, 0.000f, 0.000f, 0.000f},
+    {true, 4, 16, 16, 128, 16, 1, 2.414f, 2.021f, 1.209f, 0.007f, 0.000f, 0.000f},
+    {true, 64, 16, 16, 128, 16, 1, 1.762f, 2.505f, 1.660f, 0.000f, 0.000f, 0.000f},
+    {true, 4, 16, 32, 128, 8, 1, 2.816f, 1.105f, 1.504f, 0.066f, 0.000f, 0.000f},
+    {true, 64, 16, 32, 128, 8, 1, 2.154f, 1.603f, 2.127f, 0.048f, 0.000f, 0.000f},
+    {true, 4, 16, 32, 128, 16, 1, 1.483f, 3.549f, 1.327f, 0.075f, 0.000f, 0.000f},
+    {true, 64, 16, 32, 128, 16, 1, 1.175f, 3.178f, 2.134f, 0.046f, 0.000f, 0.000f},
+    {true, 4, 16, 64, 128, 8, 1, 0.000f, 4.249f, 1.990f, 0.092f, 0.000f, 0.000f},
+    {true, 64, 16, 64, 128, 8, 1, 0.000f, 4.341f, 2.965f, 0.084f, 0.000f, 0.000f},
 };
 
 double cost(const Candidate& c, int64_t m, int64_t n, int64_t k, int sk) {
   const double kp = (double)cdiv<int64_t>(k, 64) * 64;
-  const double rounds = std::ceil((double)cdiv<int64_t>(m, c.bm) * (double)cdiv<int64_t>(n, c.bn) * sk / 256.0);
-  double t = c.fixed + rounds * (c.round + c.step * kp / sk / 1024.0) + c.byte * 2.0 * (double)n * kp / 1e6;
+  const double rounds = (double)cdiv<int64_t>(m, c.bm) * (double)cdiv<int64_t>(n, c.bn) * sk / 256.0;
+  const double steps = kp / sk / 1024.0;
+  double t = std::max(c.fixed + std::ceil(rounds) * (c.round + c.step * steps) + c.byte * 2.0 * (double)n * kp / 1e6,
+                      rounds * (c.many_round + c.many_step * steps));
   if (!c.one_launch) t += 2.9 + (double)m * kp / 1.1e6;                      // digitize: its launch, then its bytes
   if (sk > 1) t += 2.6 + (double)m * (double)n * 8.0 * sk * 2.0 / 5e6;       // partials written and read, finalize
   return t;
