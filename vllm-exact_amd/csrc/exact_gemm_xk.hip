@@ -43,6 +43,7 @@
 namespace {
 
 typedef __attribute__((address_space(3))) void lds_void_t;
+typedef __attribute__((address_space(3))) v4i lds_v4i_t;
 
 constexpr int staged_row_bytes(int bn) { return bn * 2 + 16; }
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
@@ -132,16 +133,17 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
   // c / NFX / 2), fragment c % NFX (plane f / TM, row tile f % TM; tiles past M clamped, their
   // rows are never stored). In LDS the row tiles of group g's steps are rotated by g * TMO, so
   // that group g reads them in its accumulator order at fixed offsets.
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(lds_void_t*)ring;
   const int8_t* xsrc[LX];
-  int xstep[LX], xdst[LX];
+  uint32_t xoff[LX], xdst[LX];  // byte offset of the copy's step in a round; its place in a slot
 #pragma unroll
   for (int i = 0; i < LX; ++i) {
     const int c = (wave + NWAVE * i) % NCOPY;
     const int f = c % NFX, g = c / NFX / kSteps;
     const int64_t tile = min((int64_t)bm * TM + f % TM, last_mt);
     xsrc[i] = p.xh + (tile * p.KT + kt0) * 2048 + (f / TM) * 1024;
-    xstep[i] = c / NFX;  // = g * kSteps + s
-    xdst[i] = ((c / NFX) * NFX + (f / TM) * TM + ((f % TM - g * TMO) & (TM - 1))) * 1024;
+    xoff[i] = (uint32_t)(c / NFX) * 2048;  // step c / NFX = g * kSteps + s
+    xdst[i] = ring0 + (uint32_t)((c / NFX) * NFX + (f / TM) * TM + ((f % TM - g * TMO) & (TM - 1))) * 1024;
   }
   const int8_t* wsrc[TN];
 #pragma unroll
@@ -150,21 +152,24 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
     wsrc[tn] = p.wh + (tile * p.KT + kt0) * 2048;
   }
 
-  // x copy i of this wave for round `round` into ring slot `slot`
-  auto issue_x = [&](int round, int slot, int i) {
-    const int step = min(round * KG * kSteps + xstep[i], nk - 1);
-    const uint32_t dst = __builtin_amdgcn_readfirstlane(
-        (uint32_t)(uintptr_t)(lds_void_t*)(ring + slot * kSlot + xdst[i]));
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(xsrc[i] + step * 2048),
+  // Byte offsets of steps: round r starts at r * kRoundBytes; steps past the last repeat it. 32 bits
+  // (at most 512 steps), one scalar add and min a load.
+  constexpr uint32_t kRoundBytes = KG * kSteps * 2048;
+  const uint32_t last_off = (uint32_t)max(nk - 1, 0) * 2048;
+  // x copy i of this wave for the round at byte `at` into ring slot `slot`
+  auto issue_x = [&](uint32_t at, int slot, int i) {
+    const uint32_t off = min(at + xoff[i], last_off);
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(xdst[i] + slot * kSlot);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(xsrc[i] + off),
                  "s"(dst)
                  : "memory", "m0");
   };
-  // Weight fragment f (column tile f / 2, plane f % 2) of step s of round `round` of this wave.
+  // Weight fragment f (column tile f / 2, plane f % 2) of step s of the round at byte `at` of this wave.
   // Written by the hardware when the load completes: the registers are not read before the
   // explicit wait that covers the load.
-  auto issue_w = [&](int round, int s, v4i (&wb)[LW], int f) {
-    const int step = min((round * KG + kg) * kSteps + s, nk - 1);
-    const int8_t* base = wsrc[f >> 1] + step * 2048 + (f & 1) * 1024;
+  auto issue_w = [&](uint32_t at, int s, v4i (&wb)[LW], int f) {
+    const uint32_t off = min(at + (uint32_t)(kg * kSteps + s) * 2048, last_off);
+    const int8_t* base = wsrc[f >> 1] + off + (f & 1) * 1024;
     if constexpr (NTW)
       asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(wb[f]) : "v"(voff), "s"(base) : "memory");
     else
@@ -181,21 +186,47 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
 
   // One K step: accumulator row tile t holds the workgroup's row tile (t + kg * TMO) % TM (the
   // ring slot holds them in that order). after_tile(t) issues the loads placed after row tile t.
-  auto step_mfmas = [&](const int8_t* stage, const v4i (&wb)[LW], auto&& after_tile) {
+  // The x fragments go through XB register sets in turn, each read as early as its set is free, so
+  // that a read has several MFMAs to arrive: with three sets the next row tile's h plane is read
+  // before this tile's products and its l plane into the set this tile's h plane leaves; with two
+  // (the tiles whose accumulators leave no third) the next h plane goes into this one's set. The
+  // scheduling fences keep that order: without them the compiler read both planes of a tile just
+  // before its products, and used their sets for accumulators in between (4096 rows through 24576 x
+  // 4096 976 -> 966 us, the lm_head at 256 rows 414 -> 410: the chip's power limit takes back most
+  // of the cycles saved).
+  constexpr int XB = 4 * (NACC * TM * TN + 2 * LW) + 16 > 252 ? 2 : 3;
+  auto step_mfmas = [&](uint32_t stage, const v4i (&wb)[LW], auto&& after_tile) {
+    v4i xb[XB];
+    auto read = [&](int t, int plane) {
+      return *reinterpret_cast<const lds_v4i_t*>((uintptr_t)(stage + (plane * TM + t) * 1024));
+    };
+    auto set = [](int t, int plane) { return (2 * t + plane) % XB; };
+    xb[0] = read(0, 0);
+    xb[1] = read(0, 1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < TM; ++t) {
-      const int8_t* frag = stage + t * 1024;
-      const v4i xh = *reinterpret_cast<const v4i*>(frag);
-      const v4i xl = *reinterpret_cast<const v4i*>(frag + TM * 1024);
+      const bool more = t + 1 < TM;
+      if (XB == 3 && more) xb[set(t + 1, 0)] = read(t + 1, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      const v4i xh = xb[set(t, 0)];
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) acc[0][t][tn] = mfma_i8(xh, wb[2 * tn], acc[0][t][tn]);
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) acc[1][t][tn] = mfma_i8(xh, wb[2 * tn + 1], acc[1][t][tn]);
+      __builtin_amdgcn_sched_barrier(0);
+      const v4i xl = xb[set(t, 1)];
+      if (more) xb[XB == 3 ? set(t + 1, 1) : set(t + 1, 0)] = read(t + 1, XB == 3 ? 1 : 0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) acc[1][t][tn] = mfma_i8(xl, wb[2 * tn], acc[1][t][tn]);
       if constexpr (!TRUNC) {
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) acc[NACC - 1][t][tn] = mfma_i8(xl, wb[2 * tn + 1], acc[NACC - 1][t][tn]);
+      }
+      if (XB == 2) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) xb[set(t + 1, 1)] = read(t + 1, 1);
       }
       after_tile(t);
     }
@@ -211,11 +242,10 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
     for (int f = 0; f < LW; ++f) issue_w(0, 0, w0, f);
 #pragma unroll
     for (int f = 0; f < LW; ++f) issue_w(0, 1, w1, f);
-    const int8_t* lds_lane = ring + kg * kSteps * NFX * 1024 + lane * 16;
+    uint32_t stage = ring0 + kg * kSteps * NFX * 1024 + voff;  // this lane's x of round r, in place
     for (int r = 0; r < nr; ++r) {
       const int slot = r & 1;
-      const int nxt = tail > 0 || r + 1 < nr ? r + 1 : nr - 1;  // steps past the end are clamped
-      const int8_t* stage = lds_lane + slot * kSlot;
+      const uint32_t nxt = (uint32_t)(r + 1) * kRoundBytes;
       // x(r) landed (younger: W0(r), W1(r)); every wave is done with the slot of round r - 1
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * LW) : "memory");
       // W0(r) landed (younger: W1(r))
@@ -234,11 +264,11 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
       });
 #pragma unroll
       for (int f = 0; f < LW; ++f) issue_w(nxt, 1, w1, f);
+      stage += slot ? -kSlot : kSlot;
     }
     // the loads past the last round (repeats of its last step, or the round K ends in) have landed
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (tail > 0) {
-      const int8_t* stage = lds_lane + (nr & 1) * kSlot;
       if (kg * kSteps < tail) step_mfmas(stage, w0, [](int) {});
       if (kg * kSteps + 1 < tail) step_mfmas(stage + NFX * 1024, w1, [](int) {});
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the ring is free
