@@ -31,8 +31,8 @@
 // exchanges between lane rows are lane swaps and DPP operands instead of LDS round trips; where
 // a page holds whole tiles, a row address is a scalar base and a lane offset. Measured at
 // H32/KV8/D128, page 16, event-timed calls, us, K then V read per tile with LDS
-// exchanges -> this: one request of 16384 keys 88.5 -> 22.7 (units; whole segments 35.3), of 1024
-// 44.5 -> 11.4; 4 of 16384 97.0 -> 49.7 (2.8 -> 5.4 TB/s); 32 of 1024 49.6 -> 26.1; 64 of 8192
+// exchanges -> this: one request of 16384 keys 88.5 -> 21.2 (units; whole segments 35.3), of 1024
+// 44.5 -> 11.2; 4 of 16384 97.0 -> 49.7 (2.8 -> 5.4 TB/s); 32 of 1024 49.6 -> 26.1; 64 of 8192
 // 342.6 -> 339.7 (6.3 TB/s), with lengths spread over 4096..8192 298.8 -> 276.1; 256 of 1024 at
 // H16/KV2/D256, page 528: 186.5 -> 113.0. The units also shorten the fp32 sums: the error against
 // float64 fell by 18 % over 27 shapes of 64 to 16384 keys (largest 2.99e-7 -> 2.40e-7).
@@ -222,6 +222,7 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   if (p.n_live != nullptr && b >= *p.n_live) return;  // not a live request: nothing read or written
 
   const int L = p.sl[b];
+
   // Segments the request needs, capped at the model's NS as the fixed grid caps them. A grid
   // trimmed by the caller's bound on the batch's lengths covers every request within that
   // bound with the same segments (the same bits); a longer request gets NaN rows, written by
@@ -520,21 +521,27 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   }
 }
 
-// Merge of the units of one (request, head), one workgroup of 16 waves per (b, head), in the
-// order of the whole-segment kernel: wave w's units of a segment (w, w + NW, ...), the NW waves,
-// then the segments. A pass takes kSegs segments: their kSegs * NW unit chains go to the waves
-// (kBatch units loaded at once, so that a chain costs about one memory latency), the segments'
-// waves are merged by groups of D threads, and the first D threads append the segments.
-template <int D, int NW>
+// Merge of the units of one (request, head), one workgroup of 16 waves, in the order of the
+// whole-segment kernel: wave w's units of a segment (w, w + NW, ...), the NW waves, then the
+// segments. A pass takes kSegs segments: their kSegs * NW unit chains go to groups of GL lanes (kBatch
+// units loaded at once, so that a chain costs about one memory latency), the segments' waves are
+// merged side by side, and one group appends the segments. What bounds a few long requests is the
+// rate at which one CU loads (133 KB of partials per head at 16384 keys): SPLIT spreads a head's
+// dims over D / 32 workgroups while that leaves at most one per CU. One request of 16384 keys, 32
+// heads of 128: 5.8 -> 4.2 us; with 192 heads of 256 (12 requests) it would take 9.7 instead of 4.4.
+template <int D, int NW, bool SPLIT>
 __global__ __launch_bounds__(1024) void paged_merge_units_kernel(PagedParams p) {
-  constexpr int DPW = D / 64;
+  constexpr int GL = SPLIT ? 32 : 64;      // lanes of a group
+  constexpr int DPL = SPLIT ? 1 : D / 64;  // dims of a lane
+  constexpr int MD = GL * DPL;             // dims of the workgroup
   constexpr int kSegs = 8;
   constexpr int kBatch = 8;
   constexpr int kChains = kSegs * NW;
-  constexpr int kPer = kChains / 16;  // chains of a wave
-  __shared__ float c_m[kChains], c_l[kChains], c_a[kChains][D];
-  __shared__ float g_m[kSegs], g_l[kSegs], g_a[kSegs][D];
-  const int64_t bh = blockIdx.x;
+  constexpr int kGroups = 1024 / GL;
+  __shared__ float c_m[kChains], c_l[kChains], c_a[kChains][MD];
+  __shared__ float g_m[kSegs], g_l[kSegs], g_a[kSegs][MD];
+  const int64_t bh = blockIdx.x / (D / MD);
+  const int d0 = (int)(blockIdx.x % (D / MD)) * MD;
   const int b = (int)(bh / p.H);
   const int head = (int)(bh % p.H);
   if (p.n_live != nullptr && b >= *p.n_live) return;
@@ -542,70 +549,54 @@ __global__ __launch_bounds__(1024) void paged_merge_units_kernel(PagedParams p) 
   const int nsb = min((L + p.split - 1) / p.split, p.ns_model);
   if (nsb > p.ns) return;  // NaN rows, written by the partial kernel
   if (nsb <= 0 && p.ns == 1) return;  // an empty request: as the whole-segment kernel leaves it
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x % GL;
+  const int group = threadIdx.x / GL;
   const int64_t base = bh * p.ns * p.units;
-  float m = kNegInf, l = 0.0f, a = 0.0f;  // the request so far: thread d < D holds column d
+  float m = kNegInf, l = 0.0f, a = 0.0f;  // the request so far: thread d < MD holds its dim
   for (int s0 = 0; s0 < nsb; s0 += kSegs) {
     const int nseg = min(kSegs, nsb - s0);
-    // the wave's chains: c = wave + 16 q, their batches loaded together
-    float cm[kPer], cl[kPer], ca[kPer][DPW];
+    for (int c = group; c < nseg * NW; c += kGroups) {
+      const int s = s0 + c / NW;
+      const int keys = min(p.split, L - s * p.split);
+      const int nunit = (keys + kUnit - 1) / kUnit;  // of the segment; this chain: c % NW, + NW, ...
+      const int64_t u0 = base + (int64_t)s * p.units;
+      float cm = kNegInf, cl = 0.0f, ca[DPL];
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      cm[q] = kNegInf;
-      cl[q] = 0.0f;
-#pragma unroll
-      for (int j = 0; j < DPW; ++j) ca[q][j] = 0.0f;
-    }
-    for (int i0 = 0; i0 * NW < p.units; i0 += kBatch) {  // units i0 .. i0 + kBatch - 1 of each chain
-      float ms[kPer][kBatch], ls[kPer][kBatch], as_[kPer][kBatch][DPW];
-#pragma unroll
-      for (int q = 0; q < kPer; ++q) {
-        const int c = wave + 16 * q;
-        if (c >= nseg * NW) break;
+      for (int j = 0; j < DPL; ++j) ca[j] = 0.0f;
+      for (int u = c % NW; u < nunit; u += NW * kBatch) {
+        float ms[kBatch], ls[kBatch], as_[kBatch][DPL];
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
-          // a unit past the segment's last is read inside the workspace and not merged
-          const int64_t ui = base + (int64_t)(s0 + c / NW) * p.units + min((i0 + k) * NW + c % NW, p.units - 1);
-          ms[q][k] = p.mp[ui];
-          ls[q][k] = p.lp[ui];
+          // a unit past the segment's last repeats the first of the batch and is not merged
+          const int64_t ui = u0 + (u + NW * k < nunit ? u + NW * k : u);
+          ms[k] = p.mp[ui];
+          ls[k] = p.lp[ui];
 #pragma unroll
-          for (int j = 0; j < DPW; ++j) as_[q][k][j] = p.ap[ui * D + lane + 64 * j];
+          for (int j = 0; j < DPL; ++j) as_[k][j] = p.ap[ui * D + d0 + lane + GL * j];
         }
-      }
-      asm volatile("" ::: "memory");  // every load of the batch is issued before the first is used
-#pragma unroll
-      for (int q = 0; q < kPer; ++q) {
-        const int c = wave + 16 * q;
-        if (c >= nseg * NW) break;
-        const int keys = min(p.split, L - (s0 + c / NW) * p.split);
-        const int nunit = (keys + kUnit - 1) / kUnit;  // of the segment; none past the request's end
+        asm volatile("" ::: "memory");  // every load of the batch is issued before the first is used
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
-          if ((i0 + k) * NW + c % NW >= nunit) break;
-          const float m0 = cm[q], l0 = cl[q];
+          if (u + NW * k >= nunit) break;
+          const float m0 = cm, l0 = cl;
 #pragma unroll
-          for (int j = 0; j < DPW; ++j) {
-            cm[q] = m0;
-            cl[q] = l0;
-            merge_state(cm[q], cl[q], ca[q][j], ms[q][k], ls[q][k], as_[q][k][j]);
+          for (int j = 0; j < DPL; ++j) {
+            cm = m0;
+            cl = l0;
+            merge_state(cm, cl, ca[j], ms[k], ls[k], as_[k][j]);
           }
         }
       }
-    }
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int c = wave + 16 * q;
       if (lane == 0) {
-        c_m[c] = cm[q];
-        c_l[c] = cl[q];
+        c_m[c] = cm;
+        c_l[c] = cl;
       }
 #pragma unroll
-      for (int j = 0; j < DPW; ++j) c_a[c][lane + 64 * j] = ca[q][j];
+      for (int j = 0; j < DPL; ++j) c_a[c][lane + GL * j] = ca[j];
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < nseg * D; i += 1024) {
-      const int sg = i / D, d = i % D;
+    for (int i = threadIdx.x; i < nseg * MD; i += 1024) {
+      const int sg = i / MD, d = i % MD;
       float sm = kNegInf, sl = 0.0f, sa = 0.0f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) merge_state(sm, sl, sa, c_m[sg * NW + w], c_l[sg * NW + w], c_a[sg * NW + w][d]);
@@ -616,12 +607,20 @@ __global__ __launch_bounds__(1024) void paged_merge_units_kernel(PagedParams p) 
       g_a[sg][d] = sa;
     }
     __syncthreads();
-    if (threadIdx.x < D)
+    if (threadIdx.x < MD)
       for (int sg = 0; sg < nseg; ++sg) merge_state(m, l, a, g_m[sg], g_l[sg], g_a[sg][threadIdx.x]);
     // the next pass writes g_* only past its first barrier, and c_* were read before the last one
   }
-  if (threadIdx.x < D)
-    store_f32_as(p.out, p.out_dtype, (int64_t)b * p.sot + (int64_t)head * p.soh + threadIdx.x, a / l);
+  if (threadIdx.x < MD)
+    store_f32_as(p.out, p.out_dtype, (int64_t)b * p.sot + (int64_t)head * p.soh + d0 + threadIdx.x, a / l);
+}
+
+template <int D>
+void launch_merge_units(const PagedParams& pp, int64_t heads, hipStream_t st) {
+  if (D > 32 && heads * (D / 32) <= 256)
+    hipLaunchKernelGGL((paged_merge_units_kernel<D, 4, true>), dim3((unsigned)(heads * (D / 32))), dim3(1024), 0, st, pp);
+  else
+    hipLaunchKernelGGL((paged_merge_units_kernel<D, 4, false>), dim3((unsigned)heads), dim3(1024), 0, st, pp);
 }
 
 // Fixed-order merge over the segments of one (request, head); one wave per (b, head).
@@ -739,9 +738,9 @@ int64_t units_of(int64_t split) { return cdiv<int64_t>(split, kUnit); }
 
 // Whether the units of a grid of ns segments per request are computed apart. keys is the most
 // keys a request of the grid may have. Measured at H32/KV8/D128 (us a call, whole segments /
-// units, graph replay): 1 request of 512 keys 11.5 / 10.5, 1024 18.5 / 11.4, 16384 35.3 / 23.0
-// (64 workgroups of whole segments); 2 of 16384 (128) 43.6 / 37.0; 4 of 16384 (256) 49.7 / 61.3;
-// 16 of 1024 (128) 23.4 / 22.1; 32 of 1024 (256) 26.0 / 39.6. Past half the CUs the units'
+// units, graph replay): 1 request of 512 keys 11.5 / 10.5, 1024 18.5 / 11.4, 16384 35.3 / 21.2
+// (64 workgroups of whole segments); 2 of 16384 (128) 43.6 / 36.4; 4 of 16384 (256) 49.7 / 61.3;
+// 16 of 1024 (128) 23.4 / 21.6; 32 of 1024 (256) 26.0 / 39.6. Past half the CUs the units'
 // partials (an eighth of the keys' bytes, written and read back) cost more than the idle CUs.
 bool use_units(int64_t n, int64_t kv_heads, int64_t ns, int64_t keys, int64_t blk, int64_t waves) {
   return blk == 16 && waves == 4 && keys > 8 * kUnit && n * kv_heads * ns <= 128;
@@ -863,9 +862,9 @@ int paged_decode_impl(const void* q, int64_t sqt, int64_t sqh, const void* k_cac
   if (partials && blocks > 0x7FFFFFFFLL) return VXA_ERR_UNSUPPORTED;
   if (mode == kUnits) {
     switch (head_dim) {
-      case 64: hipLaunchKernelGGL((paged_merge_units_kernel<64, 4>), dim3((unsigned)blocks), dim3(1024), 0, st, pp); break;
-      case 128: hipLaunchKernelGGL((paged_merge_units_kernel<128, 4>), dim3((unsigned)blocks), dim3(1024), 0, st, pp); break;
-      default: hipLaunchKernelGGL((paged_merge_units_kernel<256, 4>), dim3((unsigned)blocks), dim3(1024), 0, st, pp); break;
+      case 64: launch_merge_units<64>(pp, blocks, st); break;
+      case 128: launch_merge_units<128>(pp, blocks, st); break;
+      default: launch_merge_units<256>(pp, blocks, st); break;
     }
     if (hipGetLastError() != hipSuccess) return VXA_ERR_LAUNCH;
   } else if (ns > 1) {
