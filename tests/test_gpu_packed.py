@@ -471,3 +471,21 @@ def test_packed_entry_points_reject_malformed_inputs():
         K.exact_linear_packed(xp, wp, 320, 14, True, cfg=cfg)   # K disagrees with the packed shape
     with pytest.raises(ValueError):
         K.digitize_packed(x.to(DEV), 14, out=(xp[0], xp[1][:3], xp[2]))
+
+
+@pytest.mark.parametrize("F,tr", [(14, True), (14, False), (12, True), (15, False)])
+@pytest.mark.parametrize("M,N,Kd", [(1, 48, 64), (3, 95, 4096), (16, 97, 2048), (5, 200, 2056), (20, 333, 1000), (2, 80, 4104)])
+def test_wide_one_launch_tiles_bitwise(F, tr, M, N, Kd):
+    """The one-launch kernel's wide x-in-registers tiles (48, 80 and 96 columns; 4 and 8 steps of x a
+    wave, and K past them, which runs a narrower tile): the oracle's bits at ragged M, N and K, rows of
+    magnitudes 1e-3 to 1e3 and a zero row."""
+    x, w = stress_xw(M, N, Kd, seed=M + Kd)
+    x = (x * (10.0 ** torch.linspace(-3, 3, M))[:, None]).to(torch.bfloat16)
+    if M >= 3:
+        x[1] = 0
+    w = w.to(torch.bfloat16)
+    ref = oracle.exact_linear_c(oracle.digitize_c(x.float().numpy(), F), oracle.digitize_c(w.float().numpy(), F), F, tr)
+    wp = K.digitize_packed(w.to(DEV), F)
+    for cfg in K.ONE_LAUNCH_WIDE:
+        y = K.exact_linear_bf16x(x.to(DEV), wp, Kd, F, tr, cfg=cfg + (1,))
+        assert np.array_equal(f32_bits(y.cpu().numpy()), f32_bits(ref)), cfg

@@ -42,6 +42,7 @@ struct ExactPlan {
   // small-M register-streaming kernel: MT x NT MFMA tiles per wave, NWK waves along K,
   // C 64-wide K steps whose loads are issued together
   int mt, nt, nwk, chunk;
+  int wide;  // column tiles of the one-launch kernel's wide tile (3, 5 or 6), or 0
   // LDS pipeline kernel: BM x BN workgroup tile, S ring stages; x-through-LDS kernel:
   // BM x BN workgroup tile, `stages` = R weight register sets, `nwk` = 3, 4, 6 or 8 waves
   int bm, bn, stages;

@@ -79,12 +79,13 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_kernel(FusedParams p) {
       r[1] = uint4{0u, 0u, 0u, 0u};
     }
   };
-  uint32_t cs = 0;  // this lane's part of its row's digit sum (F = 15; wraps like the digitize kernels)
+  // This lane's part of its row's sum of q (F = 15; wraps like the digitize kernels). The digit sum is
+  // 256 h + l = q - 128 over the K columns: the epilogue takes 128 K off. Columns past K have x = 0,
+  // q = 0: nothing here, and their nonzero offset digits meet the weights' zero padding digits.
+  uint32_t cs = 0;
   auto x_digits = [&](int64_t s, const uint4 (&r)[2], v4i& ah, v4i& al) {
     float v[16];
     const int64_t c0 = s * 64 + kq * 16;
-    // columns of this lane's 16 inside K (all 16 but in the chunk K ends in; none past it)
-    const int lim = (int)max<int64_t>(min<int64_t>(p.K - c0, 16), 0);
     if (!row_ok || c0 + 16 <= p.K) {
       const uint32_t w[8] = {r[0].x, r[0].y, r[0].z, r[0].w, r[1].x, r[1].y, r[1].z, r[1].w};
 #pragma unroll
@@ -103,12 +104,7 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_kernel(FusedParams p) {
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
         qv[b] = (int32_t)(v[4 * q + b] * scale);  // truncation toward zero
-        if constexpr (OFFSET) {
-          // columns past K keep zero digits and stay out of the sum, as in the digitize kernels:
-          // q = 128 is zero offset digits, and the sum adds 256 h + l = q - 128
-          qv[b] = 4 * q + b < lim ? qv[b] : 128;
-          cs += (uint32_t)qv[b] - 128u;
-        }
+        if constexpr (OFFSET) cs += (uint32_t)qv[b];
       }
       pack_digit_bytes<OFFSET>(qv, hw[q], lw[q]);
     }
@@ -320,7 +316,7 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_kernel(FusedParams p) {
     if (n < p.N) {
       int64_t tot = (int64_t)red[i];
       if constexpr (OFFSET) {  // 128 (cx + cw) + 128^2 K (kernels.py:96-97, 148-151)
-        uint32_t cx = 0;
+        uint32_t cx = 0u - 128u * (uint32_t)p.K;
 #pragma unroll
         for (int w = 0; w < NWK; ++w) cx += s_cs[w][m];
         tot += 128 * ((int64_t)(int32_t)cx + (int64_t)p.cw[n]) + 128 * 128 * p.K;
@@ -338,7 +334,11 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_kernel(FusedParams p) {
 // arrive during the absmax; each later round's weights are issued before the MFMAs of the
 // round before it. Needs cdiv(KT, NWK) <= XS (the launcher picks XS). OFFSET (F = 15): offset
 // digits, with each row's digit sum cx added in the epilogue (kernels.py:31-34, 96-97).
-template <int NT, int NWK, int C, bool TRUNC, int XS, bool OFFSET>
+//
+// WB: weight buffers. With one (the wide tiles of 3, 5 or 6 column tiles, whose second buffer would
+// spill) a round's weights are issued right after the round before it has used the buffer, ahead of
+// the digits of their own round.
+template <int NT, int NWK, int C, bool TRUNC, int XS, bool OFFSET, int WB>
 __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams p) {
   static_assert(XS % C == 0, "rounds of C steps");
   constexpr int BN = 16 * NT;
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
   __shared__ int32_t s_sh[16];
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = WB == 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)(threadIdx.x >> 6);
   const int r16 = lane & 15;
   const int kq = lane >> 4;
   const int nthr = 64 * NWK;
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int64_t tile = min(bn * NT + nt, cdiv<int64_t>(p.N, 16) - 1);
-    whp[nt] = p.wp + tile * p.KT * 2048 + lane * 16;
+    whp[nt] = p.wp + tile * p.KT * 2048 + (WB == 1 ? 0 : lane * 16);  // WB == 1: a scalar base, the lane below
   }
 
   // 1. x of this lane's steps, bf16 pairs as loaded (zeros past K and for rows past M).
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
   }
 
   // 2. Weights, double-buffered by round; round 0 is issued behind x.
-  v4i wh[2][C][NT], wl[2][C][NT];
+  v4i wh[WB][C][NT], wl[WB][C][NT];
   auto load_round = [&](int r, int buf) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -405,8 +405,10 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
       if (s < nsteps) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-          wh[buf][c][nt] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(whp[nt] + s * 2048));
-          wl[buf][c][nt] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(whp[nt] + s * 2048 + 1024));
+          const int8_t* w = whp[nt] + s * 2048;
+          if constexpr (WB == 1) w += (uint32_t)lane * 16;
+          wh[buf][c][nt] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(w));
+          wl[buf][c][nt] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(w + 1024));
         }
       }
     }
@@ -448,18 +450,18 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
     mx[nt] = v4i{0, 0, 0, 0};
     ll[nt] = v4i{0, 0, 0, 0};
   }
-  uint32_t cs = 0;  // this lane's part of its row's digit sum (F = 15; wraps like the digitize kernels)
+  // This lane's part of its row's sum of q (F = 15; wraps like the digitize kernels). The digit sum is
+  // 256 h + l = q - 128 over the K columns: the epilogue takes 128 K off. Columns past K have x = 0,
+  // q = 0: nothing here, and their nonzero offset digits meet the weights' zero padding digits.
+  uint32_t cs = 0;
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     if (wave + (int64_t)NWK * r * C >= nsteps) break;  // this wave has no steps left
-    if (r + 1 < NR) load_round(r + 1, (r + 1) & 1);
+    if (WB == 2 && r + 1 < NR) load_round(r + 1, (r + 1) % WB);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const int i = r * C + c;
-      const int64_t c0 = (wave + (int64_t)NWK * i) * 64 + kq * 16;  // this lane's first column
       if (wave + (int64_t)NWK * i < nsteps) {
-        // columns of this lane's 16 inside K (all 16 but in the chunk K ends in)
-        const int lim = (int)min<int64_t>(p.K - c0, 16);
         uint32_t hw[4], lw[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -469,19 +471,13 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
             const uint32_t w = xw[i][(4 * q + b) >> 1];
             const float v = __uint_as_float(((4 * q + b) & 1) ? (w & 0xFFFF0000u) : (w << 16));
             qv[b] = (int32_t)(v * scale);  // truncation toward zero
-            if constexpr (OFFSET) {
-              // columns past K keep zero digits: the weights' padding digits are zero too, and
-              // the digitize kernels leave those columns out of the sum (a select, not a branch;
-              // q = 128 is zero offset digits, and the sum adds 256 h + l = q - 128)
-              qv[b] = 4 * q + b < lim ? qv[b] : 128;
-              cs += (uint32_t)qv[b] - 128u;
-            }
+            if constexpr (OFFSET) cs += (uint32_t)qv[b];
           }
           pack_digit_bytes<OFFSET>(qv, hw[q], lw[q]);
         }
         const v4i ah = v4i{(int)hw[0], (int)hw[1], (int)hw[2], (int)hw[3]};
         const v4i al = v4i{(int)lw[0], (int)lw[1], (int)lw[2], (int)lw[3]};
-        const int buf = r & 1;
+        const int buf = r % WB;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) hh[nt] = mfma_i8(ah, wh[buf][c][nt], hh[nt]);
 #pragma unroll
@@ -497,6 +493,7 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
         }
       }
     }
+    if (WB == 1 && r + 1 < NR) load_round(r + 1, 0);
   }
 
   // 5. Wave partials meet in LDS (exact int64 adds), then the epilogue; with offset digits the
@@ -524,7 +521,7 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
     if (n < p.N) {
       int64_t tot = (int64_t)red[i];
       if constexpr (OFFSET) {  // 128 (cx + cw) + 128^2 K (kernels.py:96-97, 148-151)
-        uint32_t cx = 0;
+        uint32_t cx = 0u - 128u * (uint32_t)p.K;
 #pragma unroll
         for (int w = 0; w < NWK; ++w) cx += s_cs[w][mr];
         tot += 128 * ((int64_t)(int32_t)cx + (int64_t)p.cw[n]) + 128 * 128 * p.K;
@@ -580,7 +577,7 @@ hipError_t launch(const FusedParams& fp, hipStream_t st) {
 #define VXA_XREG(XS_, OFF_)                                                                                      \
   if constexpr (XS_ % C == 0 && xreg_fits<NT, NWK, C, XS_, TRUNC, OFF_>()) {                                \
     if (per_wave <= XS_ && (fp.F == 15) == OFF_) {                                                            \
-      hipLaunchKernelGGL((exact_fused_xreg_kernel<NT, NWK, C, TRUNC, XS_, OFF_>), dim3((unsigned)blocks),     \
+      hipLaunchKernelGGL((exact_fused_xreg_kernel<NT, NWK, C, TRUNC, XS_, OFF_, 2>), dim3((unsigned)blocks),  \
                          dim3(64 * NWK), 0, st, fp);                                                        \
       return hipGetLastError();                                                                               \
     }                                                                                                       \
@@ -602,6 +599,33 @@ hipError_t launch(const FusedParams& fp, hipStream_t st) {
   return hipErrorInvalidValue;  // offset digits with 3 dots, or a shape whose digit sum would spill
 }
 
+// The wide x-in-registers tiles: NT = 3, 5 or 6 column tiles, 8 waves, K up to 4096 columns (8
+// steps a wave), any grid. They fill the CUs where 1, 2 or 4 tiles leave a last round nearly empty
+// or some CUs idle, and read x once per 48 to 96 columns, where the row pass reads it twice per 16
+// to 64 (a CU loads bytes from L2 at ~83 KB/us, which at 16 rows costs as much as the weights of 16
+// columns). Measured at K = 4096, us, best narrower tile -> wide: N = 10240 18.3 -> 17.0 at M = 1,
+// 20.0 -> 19.1 at 16 (F = 15: 22.0 -> 19.3); N = 20480 35.4 -> 32.3 at 16 (F = 15: 38.3 -> 32.7); N
+// = 24576 37.4 -> 37.7 at 16 (F = 15: 40.2 -> 38.4). At N = 8192 and 32768, whole rounds of the
+// narrower tiles, they lose (15.3 -> 17.0, 48.0 -> 52.3 at 16). hipErrorInvalidValue where a plan names none or K is longer: the small-M
+// kernel's tile of the plan then runs.
+template <int NT, bool TRUNC>
+hipError_t launch_wide(const FusedParams& fp, hipStream_t st) {
+  const int64_t blocks = cdiv<int64_t>(fp.M, 16) * cdiv<int64_t>(fp.N, 16 * NT);
+  if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
+  const int64_t per_wave = cdiv<int64_t>(fp.KT, 8);
+#define VXA_WIDE(XS_, OFF_)                                                                                          \
+  if constexpr (!(OFF_ && TRUNC)) {                                                                                 \
+    if (per_wave <= XS_ && (fp.F == 15) == OFF_) {                                                                   \
+      hipLaunchKernelGGL((exact_fused_xreg_kernel<NT, 8, 1, TRUNC, XS_, OFF_, 1>), dim3((unsigned)blocks), dim3(512), \
+                         0, st, fp);                                                                                \
+      return hipGetLastError();                                                                                     \
+    }                                                                                                               \
+  }
+  VXA_WIDE(4, false) VXA_WIDE(8, false) VXA_WIDE(4, true) VXA_WIDE(8, true)
+#undef VXA_WIDE
+  return hipErrorInvalidValue;
+}
+
 // (NT, C, NWK): the small-M kernel's one-row-tile shapes.
 #define VXA_FUSED_TABLE(X)                                                                       \
   X(1, 1, 4) X(1, 1, 8) X(1, 1, 16) X(1, 2, 4) X(1, 2, 8) X(1, 2, 16) X(1, 4, 4) X(1, 4, 8)      \
@@ -610,6 +634,11 @@ hipError_t launch(const FusedParams& fp, hipStream_t st) {
 
 template <bool TRUNC>
 hipError_t dispatch(const ExactPlan& pl, const FusedParams& fp, hipStream_t st) {
+  hipError_t wide = hipErrorInvalidValue;
+  if (pl.wide == 3) wide = launch_wide<3, TRUNC>(fp, st);
+  if (pl.wide == 5) wide = launch_wide<5, TRUNC>(fp, st);
+  if (pl.wide == 6) wide = launch_wide<6, TRUNC>(fp, st);
+  if (wide != hipErrorInvalidValue) return wide;
 #define VXA_FUSED(NT_, C_, NWK_) \
   if (pl.nt == NT_ && pl.chunk == C_ && pl.nwk == NWK_) return launch<NT_, NWK_, C_, TRUNC>(fp, st);
   VXA_FUSED_TABLE(VXA_FUSED)

@@ -58,6 +58,12 @@ constexpr Candidate kThreeDots[] = {
     {true, 64, 16, 32, 128, 16, 1, 0.833f, 2.820f, 2.003f, 0.052f, 0.000f, 0.000f},
     {true, 4, 16, 64, 128, 8, 1, 0.000f, 3.714f, 2.001f, 0.095f, 0.000f, 0.000f},
     {true, 64, 16, 64, 128, 8, 1, 1.345f, 2.256f, 2.989f, 0.080f, 0.000f, 0.000f},
+{true, 4, 16, 48, 128, 8, 1, 2.955f, 0.000f, 1.563f, 0.098f, 0.000f, 0.000f},
+    {true, 64, 16, 48, 128, 8, 1, 3.128f, 0.000f, 1.981f, 0.091f, 0.000f, 0.000f},
+    {true, 4, 16, 80, 128, 8, 1, 0.906f, 2.809f, 2.485f, 0.083f, 0.000f, 0.000f},
+    {true, 64, 16, 80, 128, 8, 1, 0.700f, 3.839f, 2.744f, 0.080f, 0.000f, 0.000f},
+    {true, 4, 16, 96, 128, 8, 1, 0.956f, 2.951f, 2.959f, 0.085f, 0.000f, 0.000f},
+    {true, 64, 16, 96, 128, 8, 1, 0.898f, 4.277f, 3.108f, 0.082f, 0.000f, 0.000f},
 };
 
 constexpr Candidate kFourDots[] = {
@@ -86,6 +92,12 @@ constexpr Candidate kFourDots[] = {
     {true, 64, 16, 32, 128, 16, 1, 1.175f, 3.178f, 2.134f, 0.046f, 0.000f, 0.000f},
     {true, 4, 16, 64, 128, 8, 1, 0.000f, 4.249f, 1.990f, 0.092f, 0.000f, 0.000f},
     {true, 64, 16, 64, 128, 8, 1, 0.000f, 4.341f, 2.965f, 0.084f, 0.000f, 0.000f},
+    {true, 4, 16, 48, 128, 8, 1, 2.062f, 1.507f, 1.458f, 0.097f, 0.000f, 0.000f},
+    {true, 64, 16, 48, 128, 8, 1, 1.807f, 2.413f, 1.759f, 0.089f, 0.000f, 0.000f},
+    {true, 4, 16, 80, 128, 8, 1, 0.701f, 3.394f, 2.462f, 0.083f, 0.000f, 0.000f},
+    {true, 64, 16, 80, 128, 8, 1, 0.780f, 4.421f, 2.662f, 0.081f, 0.000f, 0.000f},
+    {true, 4, 16, 96, 128, 8, 1, 1.050f, 2.564f, 3.130f, 0.086f, 0.000f, 0.000f},
+    {true, 64, 16, 96, 128, 8, 1, 0.940f, 4.488f, 3.203f, 0.082f, 0.000f, 0.000f},
 };
 
 double cost(const Candidate& c, int64_t m, int64_t n, int64_t k, int sk) {
@@ -112,6 +124,8 @@ extern "C" int vxa_exact_linear_pick(int64_t m, int64_t n, int64_t k, int trunc,
   for (int i = 0; i < count; ++i) {
     const Candidate& c = set[i];
     if (m > c.max_rows || (c.one_launch && (!one_launch_ok || k > 32768))) continue;
+    const bool wide = c.one_launch && (c.bn == 48 || c.bn == 80 || c.bn == 96);
+    if (wide && k > 4096) continue;  // its x registers end there
     if (c.one_launch && i > 0 && set[i - 1].max_rows >= m && set[i - 1].one_launch && set[i - 1].bn == c.bn &&
         set[i - 1].waves == c.waves)
       continue;  // the same config's coefficients for fewer rows apply

@@ -71,7 +71,7 @@ def candidates(M, Kd):
     (kernels.py:298 filters the same way; the 32-row x-through-LDS tiles are kept for every M),
     times the split-K factors."""
     out = []
-    for c in K.EXACT_CFGS:
+    for c in K.EXACT_CFGS + (K.ONE_LAUNCH_WIDE if M <= ONE_LAUNCH_TUNE_ROWS and Kd <= 4096 else []):
         xw32 = c[2] == 64 and c[0] == 32  # the 32-row x-through-LDS tiles also serve M <= 16
         if c[0] > max(16, 1 << max(0, (M - 1).bit_length())) and not xw32:
             continue

@@ -264,6 +264,8 @@ SMALL_SHAPES = [(1, 1, 1, 4), (1, 1, 1, 8), (1, 1, 1, 16), (1, 1, 2, 4), (1, 1, 
                 (1, 4, 2, 8), (2, 1, 1, 4), (2, 1, 1, 8), (2, 1, 1, 16), (2, 1, 2, 4), (2, 1, 2, 8), (2, 2, 1, 4),
                 (2, 2, 1, 8), (2, 2, 1, 16), (2, 2, 2, 4), (2, 2, 2, 8), (2, 4, 1, 4), (2, 4, 1, 8), (4, 1, 1, 4),
                 (4, 1, 1, 8), (4, 1, 2, 4), (4, 1, 2, 8), (4, 2, 1, 4), (4, 2, 1, 8), (4, 4, 1, 4)]  # (MT, NT, C, NWK)
+# One-launch kernel only (exact_linear_bf16x; K up to 4096): wide x-in-registers tiles.
+ONE_LAUNCH_WIDE = [(16, 48, 128, 8, 1, 8), (16, 80, 128, 8, 1, 8), (16, 96, 128, 8, 1, 8)]
 LDS_SHAPES = [(64, 64, 2), (64, 64, 4), (64, 64, 8), (128, 64, 2), (128, 64, 4), (128, 64, 6), (64, 128, 2),
               (64, 128, 4), (64, 128, 6), (128, 128, 2), (128, 128, 3), (128, 128, 4)]  # (BM, BN, stages)
 XW_SHAPES = [(32, 128, 4, 4), (32, 256, 4, 4), (64, 64, 4, 4), (64, 128, 4, 4), (64, 192, 4, 4), (64, 256, 3, 4),
