@@ -48,6 +48,26 @@ def test_pack_matches_layout_and_digitize_packed(R, Kd):
         assert torch.equal(pd2, pd)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("R,Kd", [(4096, 3072), (6500, 2040), (4100, 4097), (4111, 8136), (4097, 12288), (4100, 12296)])
+def test_digitize_packed_of_many_rows(dtype, R, Kd):
+    """Many rows are digitized a 16-row tile per workgroup (4, 8 or 12 steps a wave; rows that are not
+    16-byte aligned and longer rows keep a workgroup per row): the digits, sums and shifts of the
+    row-major kernel, packed, and the oracle's on the first and last rows; zero digits in the padding."""
+    g = torch.Generator(device=DEV).manual_seed(R)
+    x = torch.randn(R, Kd, device=DEV, generator=g) * 10 ** (torch.rand(R, 1, device=DEV, generator=g) * 6 - 3)
+    x[5] = 0
+    x = x.to(dtype)
+    rows = [0, 5, R - 2, R - 1]
+    for F in (12, 14, 15):
+        packed, cs, sh = K.digitize_packed(x, F)
+        d = K.digitize(x, F)
+        want, wcs, wsh = K.pack_digits(d)
+        assert torch.equal(packed, want) and torch.equal(cs, wcs) and torch.equal(sh, wsh), F
+        o = oracle.digitize_c(x[rows].float().cpu().numpy(), F)
+        assert all(np.array_equal(a[rows].cpu().numpy(), b) for a, b in zip(d, o)), F
+
+
 @pytest.mark.parametrize("F,tr", [(14, True), (14, False), (15, False)])
 @pytest.mark.parametrize("M,N,Kd", [(1, 64, 4096), (16, 4096, 4096), (24, 384, 4096), (5, 200, 12288),
                                     (256, 1024, 4096), (300, 256, 12288), (33, 130, 1000)])
