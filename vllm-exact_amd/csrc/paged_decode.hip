@@ -192,9 +192,9 @@ constexpr int ahead_tiles() {
 }
 
 // UNITS: a workgroup computes a slice of a segment (slice_units consecutive units, the waves
-// taking them in turn) and writes each unit's partial (paged_merge_units_kernel merges them). Otherwise it computes a whole segment, each
-// wave merging its units (wave, wave + NW, ...) in order, then the waves in order. Both do the
-// same operations on the same values in the same order.
+// taking them in turn) and writes each unit's partial (paged_merge_units_kernel merges them).
+// Otherwise it computes a whole segment, each wave merging its units (wave, wave + NW, ...) in
+// order, then the waves in order. Both do the same operations on the same values in the same order.
 template <int D, int G, int TPG, int NW, bool UNITS, bool AHEAD, bool ALIGNED>
 __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   static_assert(G >= 1 && G <= 16, "GQA group must fit the 16 MFMA columns");

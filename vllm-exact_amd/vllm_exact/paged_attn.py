@@ -1,10 +1,10 @@
 """Paged decode attention with a fixed reduction order on MI355X, and the vLLM patch.
 
 Kernel (libvllm_exact_amd.so, paged_decode.hip): one workgroup per (request, KV head,
-segment of SPLIT keys), or per 256 keys of a segment when a few requests would leave the GPU
-idle (the same bits: both merge 64-key units in one order). The segment length is fixed and the segment count is fixed by the
-model's max length (paged_attn.py:3-5), so the grid is the same for every batch and the
-floating-point order of a request depends only on its own length. QK^T runs on bf16
+segment of SPLIT keys), or per WARPS units of 64 keys when a few requests would leave the GPU
+idle (the same bits: both merge the units in one order). The segment length is fixed and the
+segment count is fixed by the model's max length (paged_attn.py:3-5), so the floating-point
+order of a request depends only on its own length. QK^T runs on bf16
 matrix cores (exact products, fp32 sums); the softmax is online in base 2; P V runs in fp32.
 Segments are merged in segment order.
 
@@ -23,8 +23,8 @@ import torch
 from . import _native as _nx
 
 # gfx950 defaults, measured at H32/KV8/D128/BS16 (64x8K, 16x16K, 256x1K): one 16-key tile per
-# wave step keeps the kernel at 4 waves per SIMD, and 2048-key segments keep enough
-# workgroups in flight at 16x16K.
+# wave step, whose loads the kernel's register ring keeps in flight, and 2048-key segments keep
+# enough workgroups in flight at 16x16K.
 SPLIT = 2048
 BLK = 16
 WARPS = 4
