@@ -86,6 +86,28 @@ def test_packed_gemm_bitwise(F, tr, M, N, Kd):
     assert np.array_equal(yb.cpu().view(torch.int16).numpy().view(np.uint16), want_b)
 
 
+@pytest.mark.parametrize("F,tr", [(14, True), (15, False)])
+@pytest.mark.parametrize("M,N", [(1, 1), (3, 2), (17, 511), (16, 514), (49, 514), (64, 1025)])
+def test_split_k_finalize_bitwise(F, tr, M, N):
+    """The finalize reads partials by rows, one column a lane (odd N) or two, or by 16x16 tiles (the
+    LDS-ring and K-split kernels where the padded tiles fit the plan's workspace), 2, 4 or 8 splits
+    at once (more in passes): every split count's remainder, at the edges of a workgroup's columns."""
+    Kd = 2304
+    x, w = stress_xw(M, N, Kd, seed=M + N)
+    xd, wd = K.digitize(x.to(DEV), F), K.digitize(w.to(DEV), F)
+    ref = oracle.exact_linear_c(np_digits(xd), np_digits(wd), F, tr)
+    want_b = oracle.bf16_rne_c(ref).reshape(M, N)
+    xp, wp = K.pack_digits(xd), K.pack_digits(wd)
+    for base, sk in itertools.product(((16, 16, 128, 4, 1, 8), (64, 64, 128, 4, 4, 8), (64, 64, 256, 8, 2, 8),
+                                       (128, 128, 128, 8, 2, 8)), (2, 3, 5, 6, 9, 18)):
+        cfg = base + (sk,)
+        y = K.exact_linear_packed(xp, wp, Kd, F, tr, cfg=cfg)
+        assert np.array_equal(f32_bits(y.cpu().numpy()), f32_bits(ref)), cfg
+        yb = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+        K.exact_linear_packed(xp, wp, Kd, F, tr, out=yb, cfg=cfg)
+        assert np.array_equal(yb.cpu().view(torch.int16).numpy().view(np.uint16), want_b), cfg
+
+
 @pytest.mark.parametrize("tr", [True, False])
 def test_xw_two_byte_outputs_every_tile(tr):
     """The x-through-LDS kernels write a 2-byte output without a K split through an LDS-staged

@@ -8,37 +8,134 @@ namespace {
 
 // Split-K finalize: sum the int64 partials of every split in a fixed order (any order gives
 // the same integer), add the offset terms once, apply the epilogue (kernels.py:159-177).
-// Grid: x over column pairs (two outputs a lane, one 16-byte load a split when N is even),
-// y over rows (grid-stride past 65535 rows).
+// Grid: x over the columns, P to a lane (2 where N is even and the partials 16-byte aligned: one
+// 16-byte load a split), y over rows (grid-stride past 65535 rows). The grid is resident at once,
+// so its time is its longest chain of loads: the scales and the partials of S splits (a split past
+// the last repeats the last and counts as 0) are loaded together, where a loop over the splits
+// waited for each and then for the scales: 0.5-1 us less per call.
 constexpr int kFinThreads = 256;
+constexpr int kFinSplits = 8;  // splits loaded together at most
+template <int S, int P>
 __global__ __launch_bounds__(kFinThreads) void exact_finalize_kernel(ExactParams p) {
   const int64_t mn = p.M * p.N;
-  const int64_t n0 = ((int64_t)blockIdx.x * kFinThreads + threadIdx.x) * 2;
-  if (n0 >= p.N) return;
-  const bool two = n0 + 1 < p.N;
-  const bool vec = (p.N & 1) == 0 && ((uintptr_t)p.ws & 15) == 0;  // every pair 16-byte aligned
+  const int64_t n = ((int64_t)blockIdx.x * kFinThreads + threadIdx.x) * P;
+  if (n >= p.N) return;
+  struct alignas(8 * P) Pair {
+    int64_t t[P];
+  };
+  const int32_t* rows = p.offset ? p.cx : p.sx;  // digit sums, read (and left unused) without a branch
+  const int32_t* cols = p.offset ? p.cw : p.sw;
   for (int64_t m = blockIdx.y; m < p.M; m += gridDim.y) {
-    const int64_t idx = m * p.N + n0;
-    int64_t t0 = 0, t1 = 0;
-    if (vec) {
-      for (int s = 0; s < p.sk; ++s) {
-        const longlong2 v = *reinterpret_cast<const longlong2*>(p.ws + s * mn + idx);
-        t0 += v.x;
-        t1 += v.y;
-      }
-    } else {
-      for (int s = 0; s < p.sk; ++s) {
-        t0 += p.ws[s * mn + idx];
-        if (two) t1 += p.ws[s * mn + idx + 1];
-      }
+    int32_t sx = p.sx[m], cx = rows[m], sw[P], cw[P];
+#pragma unroll
+    for (int c = 0; c < P; ++c) {
+      sw[c] = p.sw[n + c];
+      cw[c] = cols[n + c];
     }
-    if (p.offset) t0 += offset_terms(p, m, n0);
-    store_f32_as(p.out, p.out_dtype, m * p.ldo + n0, exact_epilogue(t0, p.sx[m], p.sw[n0]));
-    if (two) {
-      if (p.offset) t1 += offset_terms(p, m, n0 + 1);
-      store_f32_as(p.out, p.out_dtype, m * p.ldo + n0 + 1, exact_epilogue(t1, p.sx[m], p.sw[n0 + 1]));
+    const int64_t* w = p.ws + m * p.N + n;
+    int64_t t[P] = {};
+    auto add = [&](int s0) {
+      Pair v[S];
+#pragma unroll
+      for (int i = 0; i < S; ++i) v[i] = *reinterpret_cast<const Pair*>(w + min(s0 + i, p.sk - 1) * mn);
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" : "+v"(sx), "+v"(cx));  // or the row's values are loaded after the sums
+#pragma unroll
+      for (int i = 0; i < S; ++i)
+#pragma unroll
+        for (int c = 0; c < P; ++c) t[c] += s0 + i < p.sk ? v[i].t[c] : 0;
+    };
+    add(0);
+    if constexpr (S == kFinSplits)
+      for (int s0 = S; s0 < p.sk; s0 += S) add(s0);
+#pragma unroll
+    for (int c = 0; c < P; ++c) {
+      if (p.offset) t[c] += offset_terms(cx, cw[c], p.K);
+      store_f32_as(p.out, p.out_dtype, m * p.ldo + n + c, exact_epilogue(t[c], sx, sw[c]));
     }
   }
+}
+
+// The same over partials in tiles (store_partial_tile): a wave to a 16x16 tile, 4 rows of a column
+// to a lane.
+template <int S, bool TRUNC>
+__global__ __launch_bounds__(kFinThreads) void exact_finalize_tiles_kernel(ExactParams p) {
+  using Hi = partial_hi_t<TRUNC>;
+  const int64_t tiles = partial_tiles(p), nt = (int64_t)blockIdx.x * (kFinThreads / 64) + threadIdx.x / 64;
+  const int64_t tile = blockIdx.y * cdiv<int64_t>(p.N, 16) + nt;
+  const int lane = threadIdx.x & 63;
+  const int64_t m0 = (int64_t)blockIdx.y * 16 + (lane >> 4) * 4, n = nt * 16 + (lane & 15);
+  if (n >= p.N || m0 >= p.M) return;
+  const int32_t* rows = p.offset ? p.cx : p.sx;  // digit sums, read (and left unused) without a branch
+  const int32_t* cols = p.offset ? p.cw : p.sw;
+  int32_t sx[4], cx[4], sw = p.sw[n], cw = cols[n];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int64_t m = min(m0 + r, p.M - 1);
+    sx[r] = p.sx[m];
+    cx[r] = rows[m];
+  }
+  const v4i* lo = reinterpret_cast<const v4i*>(p.ws) + (tile << 6) + lane;
+  const Four<Hi>* hi = reinterpret_cast<const Four<Hi>*>(reinterpret_cast<const int8_t*>(p.ws) + ((p.sk * tiles) << 10)) +
+                       (tile << 6) + lane;
+  int64_t t[4] = {};
+  auto add = [&](int s0) {
+    v4i l[S];
+    Four<Hi> h[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      const int64_t at = min(s0 + i, p.sk - 1) * (tiles << 6);
+      l[i] = lo[at];
+      h[i] = hi[at];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(sx[r]), "+v"(cx[r]));  // not loaded after the sums
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        t[r] += s0 + i < p.sk ? (int64_t)(((uint64_t)(int64_t)h[i].v[r] << 32) | (uint32_t)l[i][r]) : 0;
+  };
+  add(0);
+  if constexpr (S == kFinSplits)
+    for (int s0 = S; s0 < p.sk; s0 += S) add(s0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (m0 + r >= p.M) break;
+    int64_t tot = TRUNC ? t[r] * 256 : t[r];
+    if (p.offset) tot += offset_terms(cx[r], cw, p.K);
+    store_f32_as(p.out, p.out_dtype, (m0 + r) * p.ldo + n, exact_epilogue(tot, sx[r], sw));
+  }
+}
+
+template <bool TRUNC>
+void launch_finalize_tiles(const ExactParams& ep, hipStream_t st) {
+  const dim3 grid((unsigned)cdiv<int64_t>(ep.N, kFinThreads / 4), (unsigned)cdiv<int64_t>(ep.M, 16)), block(kFinThreads);
+  if (ep.sk <= 2)
+    hipLaunchKernelGGL((exact_finalize_tiles_kernel<2, TRUNC>), grid, block, 0, st, ep);
+  else if (ep.sk <= 4)
+    hipLaunchKernelGGL((exact_finalize_tiles_kernel<4, TRUNC>), grid, block, 0, st, ep);
+  else
+    hipLaunchKernelGGL((exact_finalize_tiles_kernel<kFinSplits, TRUNC>), grid, block, 0, st, ep);
+}
+
+// Whether the partials go in tiles: where the kernel's accumulators are whole tiles, and the
+// padded tiles fit the workspace of int64 [sk][M][N] that a plan asks for (and the finalize's grid).
+bool tiled_partials(const ExactParams& ep, bool trunc) {
+  return ep.sk > 1 && partial_tiles(ep) * 256 * (trunc ? 5 : 6) <= ep.M * ep.N * 8 && (uintptr_t)ep.ws % 16 == 0 &&
+         ep.M <= 65535 * 16;
+}
+
+template <int P>
+void launch_finalize(const ExactParams& ep, unsigned by, hipStream_t st) {
+  const dim3 grid((unsigned)cdiv<int64_t>(ep.N, P * kFinThreads), by), block(kFinThreads);
+  if (ep.sk <= 2)
+    hipLaunchKernelGGL((exact_finalize_kernel<2, P>), grid, block, 0, st, ep);
+  else if (ep.sk <= 4)
+    hipLaunchKernelGGL((exact_finalize_kernel<4, P>), grid, block, 0, st, ep);
+  else
+    hipLaunchKernelGGL((exact_finalize_kernel<kFinSplits, P>), grid, block, 0, st, ep);
 }
 
 // Slow path for shapes the vector kernels do not take (K not a multiple of 64, rows not
@@ -163,7 +260,8 @@ namespace {
 // Launch the GEMM kernels (and the split-K finalize) for a filled-in ExactParams.
 int run_exact(const ExactPlan& pl, ExactParams& ep, int trunc, bool packed, bool vec_ok, hipStream_t st) {
   hipError_t err;
-  const int64_t fin_bx = cdiv<int64_t>(ep.N, 2 * kFinThreads);  // finalize grid: column pairs x rows
+  ep.tiled = 0;
+  const int64_t fin_bx = cdiv<int64_t>(ep.N, kFinThreads);  // finalize grid: columns (or pairs) x rows
   const int64_t fin_by = ep.M < 65535 ? ep.M : 65535;
   if (pl.sk > 1 && fin_bx > 0x7FFFFFFFLL) return VXA_ERR_UNSUPPORTED;
   if (!vec_ok) {
@@ -174,6 +272,7 @@ int run_exact(const ExactPlan& pl, ExactParams& ep, int trunc, bool packed, bool
   } else if (pl.family == kFamilyXw && packed && exact_xw_supported(pl.bm, pl.bn, pl.stages, pl.nwk, trunc != 0)) {
     err = launch_exact_xw(pl, ep, trunc != 0, st);
   } else if (pl.family == kFamilyXk && packed && exact_xk_supported(pl.bm, pl.bn, pl.kg, pl.stages, pl.nwk, trunc != 0)) {
+    ep.tiled = tiled_partials(ep, trunc != 0);
     err = launch_exact_xk(pl, ep, trunc != 0, st);
   } else if (pl.family == kFamilyXw || pl.family == kFamilyXk || pl.family == kFamilyLds) {
     ExactPlan lp = pl;
@@ -182,6 +281,7 @@ int run_exact(const ExactPlan& pl, ExactParams& ep, int trunc, bool packed, bool
       lp.bn = pl.bn >= 128 ? 128 : 64;
       lp.stages = lds_stages(lp.bm, lp.bn, 4);
     }
+    ep.tiled = tiled_partials(ep, trunc != 0);
     err = launch_exact_lds(lp, ep, trunc != 0, packed, st);
   } else {
     err = launch_exact_small(pl, ep, trunc != 0, packed, st);
@@ -189,8 +289,14 @@ int run_exact(const ExactPlan& pl, ExactParams& ep, int trunc, bool packed, bool
   if (err == hipErrorInvalidValue) return VXA_ERR_UNSUPPORTED;
   if (err != hipSuccess) return VXA_ERR_LAUNCH;
   if (pl.sk > 1) {
-    hipLaunchKernelGGL(exact_finalize_kernel, dim3((unsigned)fin_bx, (unsigned)fin_by), dim3(kFinThreads), 0, st,
-                       ep);
+    if (ep.tiled && trunc)
+      launch_finalize_tiles<true>(ep, st);
+    else if (ep.tiled)
+      launch_finalize_tiles<false>(ep, st);
+    else if (ep.N % 2 == 0 && (uintptr_t)ep.ws % 16 == 0)
+      launch_finalize<2>(ep, (unsigned)fin_by, st);
+    else
+      launch_finalize<1>(ep, (unsigned)fin_by, st);
     if (hipGetLastError() != hipSuccess) return VXA_ERR_LAUNCH;
   }
   return VXA_OK;

@@ -142,6 +142,16 @@ __global__ __launch_bounds__(256) void exact_lds_kernel(ExactParams p) {
   }
 
   // Epilogue from registers: register r of lane holds C[4*(lane>>4) + r][lane & 15].
+  if (p.tiled) {
+    const int64_t mt = (m0 + wm * (BM / 2)) / 16, nt = (n0 + wn * (BN / 2)) / 16;
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+        store_partial_tile<TRUNC>(p, blockIdx.y, mt + tm, nt + tn, lane, hh[tm][tn], md[tm][tn],
+                                  TRUNC ? hh[tm][tn] : ll[tm][tn]);
+    return;
+  }
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
 #pragma unroll

@@ -32,7 +32,8 @@
 // hold the row tiles it owns after the K loop, [g * TM / KG, (g + 1) * TM / KG): one copy of
 // the reduction and epilogue code serves every group. The K groups reduce in LDS, then the
 // owner applies the epilogue to its rows: for 2-byte outputs without a K split or offset terms
-// (STAGED) through an LDS tile stored in 16-byte pieces of whole rows, otherwise lane by lane.
+// (STAGED) through an LDS tile stored in 16-byte pieces of whole rows, a K split's partials as
+// whole MFMA tiles where they fit the workspace (store_partial_tile), otherwise lane by lane.
 // The row and column scales were copied into LDS at the start. Integer addition is exact and
 // associative, so the bits are those of every other kernel.
 
@@ -388,6 +389,15 @@ __global__ __launch_bounds__(64 * NWN * KG) void exact_xk_kernel(ExactParams p) 
         for (int e = 0; e < 8 && n + e < p.N; ++e) dst[e] = reinterpret_cast<const uint16_t*>(src)[e];
       }
     }
+    return;
+  }
+  if (p.tiled) {
+#pragma unroll
+    for (int t = 0; t < TMO; ++t)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+        store_partial_tile<TRUNC>(p, split, m0 / 16 + kg * TMO + t, n0 / 16 + tn, lane, acc[0][t][tn], acc[1][t][tn],
+                                  acc[NACC - 1][t][tn]);
     return;
   }
 #pragma unroll
