@@ -308,3 +308,28 @@ def test_units_and_whole_segments_give_the_same_bits(monkeypatch, D, H, KV, BS, 
             a, c = run(b, True, bound, live), run(b, False, bound, live)
             assert torch.equal(a.view(torch.int32), c.view(torch.int32)), (lens[b], bound, live)
     assert any(took) == (2 * KV * -(-700 // split) <= 128)  # the grids that take units
+
+
+@pytest.mark.parametrize("blk,waves,split", [(16, 4, 2048), (16, 4, 528), (32, 8, 2048), (64, 4, 512)])
+@pytest.mark.parametrize("BS", [16, 24])
+def test_keys_that_score_minus_infinity_weigh_nothing(monkeypatch, BS, blk, waves, split):
+    """Keys whose score is -inf (a cache row holding -inf) have weight 0 wherever they lie: the first
+    tile of a unit, whole units, a wave's first unit, whole segments, the last partial tile. With
+    units in workgroups of their own and in whole segments, against the torch statement."""
+    B, H, KV, D, L = 5, 8, 2, 128, 1500
+    q, kv, bt, sl = make_paged(B, L, BS, H, KV, D, seed=41)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    sl = torch.tensor([1500, 1500, 1345, 700, 130], dtype=torch.int32)
+    spans = [[(64, 80), (512, 576)], [(0, 528), (1024, 1088)], [(1337, 1345)], [(0, 16), (64, 128), (256, 700)], [(0, 129)]]
+    kc, vc = kv_views(kv, D)
+    for b, rows in enumerate(spans):
+        for lo, hi in rows:
+            t = torch.arange(lo, hi)
+            kc[bt[b].long()[t // BS], t % BS, :, 0] = float("-inf")
+    want = P.paged_decode_torch(q, kc, vc, bt, sl, 0.09, B).numpy()
+    assert np.isfinite(want).all()
+    gpu = [t.to(DEV) for t in (q, kv, bt, sl)]
+    whole = _run(*gpu, 0.09, B, D, blk=blk, warps=waves, split=split)
+    monkeypatch.setattr(P._nx, "paged_units_workspace", lambda n, H, KV, *a: P._nx.paged_workspace(n, H, *a[:-2]))
+    assert torch.equal(_run(*gpu, 0.09, B, D, blk=blk, warps=waves, split=split).view(torch.int32), whole.view(torch.int32))
+    _check_tol(whole.cpu().numpy(), want)

@@ -366,13 +366,16 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[t][r]);
       const float m_new = fmaxf(m_run, rows_max(mx));
-      const float alpha = exp2_hw(m_run - m_new);  // m_run == -inf -> 0
+      // Where every score so far is -inf (m_new too), the differences are taken to 0: the keys weigh 0
+      // and the state stays (-inf, 0, 0), which a later merge drops; -inf - -inf would be NaN.
+      const float m_ref = (m_new == kNegInf) ? 0.0f : m_new;
+      const float alpha = exp2_hw(m_run - m_ref);  // m_run == -inf -> 0
       float psum = 0.0f;
 #pragma unroll
       for (int t = 0; t < TPG; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          sc[t][r] = exp2_hw(sc[t][r] - m_new);
+          sc[t][r] = exp2_hw(sc[t][r] - m_ref);
           psum += sc[t][r];
         }
       l_run = fmaf(l_run, alpha, rows_sum(psum));
