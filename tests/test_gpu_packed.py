@@ -205,6 +205,39 @@ def test_op_without_a_table_entry(monkeypatch, dtype, M, N, Kd):
         assert np.array_equal(y.view(torch.int16).numpy().view(np.uint16), want), (F, plugin._packed_plan(M, N, Kd, dtype))
 
 
+@pytest.mark.parametrize("M,N,Kd,offset", [(1, 5000, 1001, 0), (8, 5000, 1001, 0), (33, 7615, 826, 0), (64, 12001, 826, 0),
+                                            (8, 5000, 2601, 0), (16, 5000, 1024, 1), (8, 12288, 4096, 1)])
+def test_rows_that_cannot_take_one_launch_are_planned_for_two(monkeypatch, M, N, Kd, offset):
+    """bf16 rows that are not 16-byte aligned (K not a multiple of 8, or a view at an odd element) go
+    straight to the two launches in one native call, with the config that serves two launches, and
+    keep their plan; aligned rows of the same sizes have their own. The oracle's bits in both."""
+    plugin.load_table(vllm_exact.TABLES["mi355x"])
+    try:
+        x, w = stress_xw(M, N, Kd, seed=M + Kd)
+        x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
+        wbuf = plugin.pack_weight(w.to(DEV))
+        xg = torch.empty(M * Kd + 8, device=DEV, dtype=torch.bfloat16)[offset:offset + M * Kd].view(M, Kd).copy_(x)
+        calls = []
+        native = plugin._nx.launch
+        monkeypatch.setattr(plugin._nx, "launch", lambda *a: calls.append(a[1].__name__) or native(*a))
+        monkeypatch.setattr(plugin, "_linear_body", lambda *a: pytest.fail("the general body ran"))
+        rows = sorted({0, M // 2, M - 1})
+        ref = oracle.exact_linear_c(oracle.digitize_c(x[rows].float().numpy(), plugin.F),
+                                    oracle.digitize_c(w.float().numpy(), plugin.F), plugin.F, plugin.TRUNC)
+        want = oracle.bf16_rne_c(ref).reshape(len(rows), N)
+        for _ in range(2):
+            y = torch.ops.exactmm.linear(xg, *wbuf)
+            assert np.array_equal(y[rows].cpu().view(torch.int16).numpy().view(np.uint16), want)
+        assert calls == ["vxa_exact_linear_op"] * 2
+        assert len(plugin._PLANS) == 1
+        if Kd % 8 == 0:
+            y = torch.ops.exactmm.linear(x.to(DEV), *wbuf)
+            assert np.array_equal(y[rows].cpu().view(torch.int16).numpy().view(np.uint16), want)
+            assert calls[2:] == ["vxa_exact_linear_bf16x"] and len(plugin._PLANS) == 2
+    finally:
+        plugin.load_table(None)
+
+
 FUSED_CFGS = tuple((16, 16 * nt, 128, nwk, c, 8, 1) for mt, nt, c, nwk in K.SMALL_SHAPES if mt == 1)
 
 

@@ -56,6 +56,24 @@ def test_one_launch_marks(tmp_path):
     assert plugin._one_launch(4, 4096, 4096) and not plugin._one_launch(16, 4096, 4096)
 
 
+@pytest.mark.parametrize("M,N,Kd", [(1, 5000, 1001), (8, 5000, 1001), (32, 12001, 826), (64, 5000, 1024), (8, 5000, 2601)])
+def test_packed_plan_where_one_launch_cannot_run(M, N, Kd):
+    """Rows that are not aligned, rows of another type, and a config that one launch refused get the
+    plan the library makes for two launches, not a one-launch tile in two launches."""
+    plugin.load_table(None)
+    two = plugin._nx.exact_pick(M, N, Kd, plugin.TRUNC, False)
+    assert not two[1]
+    assert plugin._packed_plan(M, N, Kd, torch.bfloat16, aligned=False) == two
+    assert plugin._packed_plan(M, N, Kd, torch.float16) == two
+    cfg, one = plugin._packed_plan(M, N, Kd, torch.bfloat16)
+    assert one
+    try:
+        plugin._ONE_LAUNCH_CFG[plugin._one_launch_key(cfg, M, N, Kd)] = False
+        assert plugin._packed_plan(M, N, Kd, torch.bfloat16) == two
+    finally:
+        plugin.load_table(None)
+
+
 def test_tuner_merge_keeps_untuned_entries():
     import importlib.util
     from pathlib import Path

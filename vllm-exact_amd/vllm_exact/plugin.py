@@ -105,18 +105,10 @@ def _n_split(M, N, Kd):
     return _N_SPLIT[(N, Kd)].get(next(m for m in ms if m >= M))
 
 
-def _packed_plan(M, N, Kd, dtype):
-    """(cfg, one launch) of a packed (M, N, K) call: the table's where it has the shape and a row
-    of at least M rows, otherwise the library's choice by size (exact_pick.hip; speed only). One
-    launch takes bf16 rows only."""
-    if _TABLE is not None and (N, Kd) in _TABLE and M <= max(_TABLE[(N, Kd)]):
-        return _cfg(M, N, Kd), dtype == torch.bfloat16 and _one_launch(M, N, Kd)
-    return _nx.exact_pick(M, N, Kd, TRUNC, dtype == torch.bfloat16)
-
-
-# (F, trunc, cfg, N, K[, M at F = 15]) the one-launch digitize + GEMM path refused. At F < 15
-# a refusal depends on the cfg and K (a K past 32768 columns needs a second K split); at F = 15
-# also on the grid, hence the row count. Cleared by load_table.
+# (F, trunc, cfg, N, K[, M at F = 15]) the one-launch digitize + GEMM path refused for another
+# reason than its rows' alignment. At F < 15 a refusal depends on the cfg and K (a K past 32768
+# columns needs a second K split); at F = 15 also on the grid, hence the row count. Cleared by
+# load_table.
 _ONE_LAUNCH_CFG = {}
 
 
@@ -124,12 +116,29 @@ def _one_launch_key(cfg, M, N, Kd):
     return (F, TRUNC, tuple(cfg), N, Kd) + ((M,) if F == 15 else ())
 
 
+def _packed_plan(M, N, Kd, dtype, aligned=True):
+    """(cfg, one launch) of a packed (M, N, K) call: the table's where it has the shape and a row
+    of at least M rows, otherwise the library's choice by size (exact_pick.hip; speed only). One
+    launch takes bf16 rows only, of 16-byte `aligned` rows (K.bf16x_rows_aligned); where it cannot
+    run, the library chooses among the configs of two launches. Rows of K = 1001 that were planned
+    for one launch and refused at every call took 62.9 us an eager call at 8 x 5000 x 1001, and take
+    17.7 this way; 32 x 12001 x 826 on the one-launch tile took 14.5 us on the GPU, and takes 11.8."""
+    one_ok = aligned and dtype == torch.bfloat16
+    if _TABLE is not None and (N, Kd) in _TABLE and M <= max(_TABLE[(N, Kd)]):
+        cfg, one_launch = _cfg(M, N, Kd), one_ok and _one_launch(M, N, Kd)
+        return cfg, one_launch and _ONE_LAUNCH_CFG.get(_one_launch_key(cfg, M, N, Kd), True)
+    cfg, one_launch = _nx.exact_pick(M, N, Kd, TRUNC, one_ok)
+    if one_launch and not _ONE_LAUNCH_CFG.get(_one_launch_key(cfg, M, N, Kd), True):
+        cfg, one_launch = _nx.exact_pick(M, N, Kd, TRUNC, False)
+    return cfg, one_launch
+
+
 def _linear_body(x: torch.Tensor, wh: torch.Tensor, wl: torch.Tensor, cw: torch.Tensor,
                  sw: torch.Tensor) -> torch.Tensor:
     """y = x @ W^T through the exact path: reshape to 2-D, digitize x (bf16 read directly),
     exact matmul straight into an x.dtype output, in row blocks of RB (plugin.py:51-64). With
-    packed weights, bf16 rows, a one-row-tile cfg and a row count the table marks (1-4 rows
-    without a mark), digitize and GEMM share one launch (same bits).
+    packed weights, 16-byte aligned bf16 rows and a plan for it (_packed_plan), digitize and GEMM
+    share one launch (same bits).
 
     Weights come either as the reference's row-major digit planes wh, wl [N, K], or packed
     at load time (wh = packed [cdiv(N,16), cdiv(K,64), 2, 1024], wl empty); N is sw's length
@@ -145,16 +154,16 @@ def _linear_body(x: torch.Tensor, wh: torch.Tensor, wl: torch.Tensor, cw: torch.
     for i in range(0, M, RB):
         xb = x2[i:i + RB]
         if packed:
-            cfg, one_launch = _packed_plan(xb.shape[0], N, Kd, xb.dtype)
-            key = _one_launch_key(cfg, xb.shape[0], N, Kd)
-            if one_launch and _ONE_LAUNCH_CFG.get(key, True):
+            aligned = K.bf16x_rows_aligned(xb)
+            cfg, one_launch = _packed_plan(xb.shape[0], N, Kd, xb.dtype, aligned)
+            if one_launch:
                 # digitize inside the GEMM launch where the cfg allows it (same bits, one launch fewer)
                 try:
                     K.exact_linear_bf16x(xb, (wh, cw, sw), Kd, F, TRUNC, out=out[i:i + RB], cfg=cfg)
                     continue
-                except NotImplementedError:
-                    if K.bf16x_rows_aligned(xb):
-                        _ONE_LAUNCH_CFG[key] = False  # refused for the cfg (and shape), not for this x
+                except NotImplementedError:  # refused for the cfg (and shape), not for this x
+                    _ONE_LAUNCH_CFG[_one_launch_key(cfg, xb.shape[0], N, Kd)] = False
+                    cfg, _ = _packed_plan(xb.shape[0], N, Kd, xb.dtype, aligned)
             xd = K.digitize_packed(xb, F)
             split = _n_split(xb.shape[0], N, Kd)
             if split is None:
@@ -179,22 +188,22 @@ def _(x, wh, wl, cw, sw):
     return x.new_empty(*x.shape[:-1], sw.shape[0])
 
 
-# (M, N, K, dtype, F, TRUNC) -> how the op runs such a packed call: (packed weight shape, one
-# launch, cfg array, its length, n1, cfg2 array, its length, scratch bytes). Sizes only; cleared by
-# load_table, and when it holds MAX_PLANS (row counts vary without bound under a server).
+# (M, N, K, dtype, F, TRUNC, aligned bf16 rows) -> how the op runs such a packed call: (packed weight
+# shape, one launch, cfg array, its length, n1, cfg2 array, its length, scratch bytes). Sizes and
+# alignment only; cleared by load_table, and when it holds MAX_PLANS (row counts vary without bound
+# under a server).
 _PLANS = {}
 MAX_PLANS = 4096
 
 
-def _op_plan(M, N, Kd, dtype):
-    cfg, one_launch = _packed_plan(M, N, Kd, dtype)
-    one_launch = one_launch and _ONE_LAUNCH_CFG.get(_one_launch_key(cfg, M, N, Kd), True)
+def _op_plan(M, N, Kd, dtype, aligned):
+    cfg, one_launch = _packed_plan(M, N, Kd, dtype, aligned)
     n1, cfg2 = _n_split(M, N, Kd) or (0, None)
     arr, n, arr2, n2, scratch = _nx.op_scratch(M, N, Kd, cfg, n1, cfg2)
     if len(_PLANS) >= MAX_PLANS:
         _PLANS.clear()
     plan = (torch.Size(K.packed_shape(N, Kd)), one_launch, arr, n, n1, arr2, n2, scratch)
-    _PLANS[(M, N, Kd, dtype, F, TRUNC)] = plan
+    _PLANS[(M, N, Kd, dtype, F, TRUNC, aligned)] = plan
     return plan
 
 
@@ -218,27 +227,30 @@ def _linear_cuda(x, wh, wl, cw, sw):
                 and sw.get_device() == index and wh.dtype == torch.int8 and cw.dtype == torch.int32
                 and sw.dtype == torch.int32 and cw.numel() == N and wh.is_contiguous() and cw.is_contiguous()
                 and sw.is_contiguous()):
-            plan = _PLANS.get((M, N, Kd, dtype, F, TRUNC)) or _op_plan(M, N, Kd, dtype)
+            # a one-row tensor may have any row stride: it is never used
+            ldx = x2.stride(0) if M > 1 else max(x2.stride(0), Kd)
+            xptr = x2.data_ptr()
+            aligned = dtype == torch.bfloat16 and xptr % 16 == 0 and ldx % 8 == 0
+            plan = _PLANS.get((M, N, Kd, dtype, F, TRUNC, aligned)) or _op_plan(M, N, Kd, dtype, aligned)
             shape, one_launch, arr, n, n1, arr2, n2, scratch = plan
             if wh.shape == shape:
                 out = x2.new_empty(M, N)
                 L = _nx.lib()
                 enum = _nx.DTYPE_ENUM[dtype]
-                # a one-row tensor may have any row stride: it is never used
-                ldx = x2.stride(0) if M > 1 else max(x2.stride(0), Kd)
                 if one_launch:
-                    status = _nx.launch(x.device, L.vxa_exact_linear_bf16x, x2.data_ptr(), ldx, wh.data_ptr(),
+                    status = _nx.launch(x.device, L.vxa_exact_linear_bf16x, xptr, ldx, wh.data_ptr(),
                                         cw.data_ptr(), sw.data_ptr(), out.data_ptr(), enum, N, M, N, Kd, F, int(TRUNC),
                                         arr, n)
                 else:
                     ws = x2.new_empty(scratch, dtype=torch.uint8)
-                    status = _nx.launch(x.device, L.vxa_exact_linear_op, x2.data_ptr(), enum, ldx, wh.data_ptr(),
+                    status = _nx.launch(x.device, L.vxa_exact_linear_op, xptr, enum, ldx, wh.data_ptr(),
                                         cw.data_ptr(), sw.data_ptr(), out.data_ptr(), enum, N, M, N, Kd, F, int(TRUNC),
                                         arr, n, n1, arr2, n2, ws.data_ptr(), scratch)
                 if status == _nx.VXA_OK:
                     return out if len(shp) == 2 else out.reshape(*shp[:-1], N)
                 if one_launch and status == _nx.VXA_ERR_UNSUPPORTED:
-                    _PLANS.pop((M, N, Kd, dtype, F, TRUNC), None)  # planned anew once the general body knows why
+                    # planned anew once the general body knows why
+                    _PLANS.pop((M, N, Kd, dtype, F, TRUNC, aligned), None)
                 else:
                     _nx.check(status, "exactmm::linear")
     return _linear_body(x, wh, wl, cw, sw)
