@@ -564,3 +564,18 @@ def test_wide_one_launch_tiles_bitwise(F, tr, M, N, Kd):
     for cfg in K.ONE_LAUNCH_WIDE:
         y = K.exact_linear_bf16x(x.to(DEV), wp, Kd, F, tr, cfg=cfg + (1,))
         assert np.array_equal(f32_bits(y.cpu().numpy()), f32_bits(ref)), cfg
+
+
+@pytest.mark.parametrize("F,tr", [(14, True), (15, False)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,Kd", [(1, 49, 4096), (7, 96, 1001), (16, 337, 4104)])
+def test_wide_tile_configs_in_two_launches_bitwise(F, tr, dtype, M, N, Kd):
+    """A wide one-launch tile's config serves the calls that take two launches (fp16 rows, unaligned
+    bf16 rows) with a narrower tile: the oracle's bits, also where K is past the wide tiles' registers."""
+    x, w = stress_xw(M, N, Kd, seed=M + Kd)
+    x, w = x.to(dtype), w.to(torch.bfloat16)
+    ref = oracle.exact_linear_c(oracle.digitize_c(x.float().numpy(), F), oracle.digitize_c(w.float().numpy(), F), F, tr)
+    wp = K.digitize_packed(w.to(DEV), F)
+    for cfg in K.ONE_LAUNCH_WIDE:
+        y = K.exact_linear_packed(K.digitize_packed(x.to(DEV), F), wp, Kd, F, tr, cfg=cfg + (1,))
+        assert np.array_equal(f32_bits(y.cpu().numpy()), f32_bits(ref)), cfg

@@ -187,7 +187,10 @@ int lds_stages(int bm, int bn, int want) {
 //   otherwise the small-M kernel: MT = BM/16 and NT = BN/16 (each clamped to 1, 2, 4),
 //     NWK = warps (4, 8, 16), C = stages (1, 2, 4), reduced to the nearest instantiated
 //     combination (fewer waves first, then a shorter chunk). BM <= 16, BN = 48, 80 or 96, warps 8,
-//     stages 1 names the one-launch kernel's wide tiles besides (vxa_exact_linear_bf16x).
+//     stages 1 names the one-launch kernel's wide tiles (vxa_exact_linear_bf16x); rows that take two
+//     launches (fp16, unaligned) run 16 columns (BN 48) or 32 (80, 96) and 4 waves there. Measured at
+//     16 fp16 rows, K = 4096, us, 64 columns and 8 waves -> this: N = 10240 25.9 -> 21.6 (F = 15: 24.8
+//     -> 22.7), 12288 28.4 -> 25.8 (27.6 -> 25.8), 24576 F = 15 (BN 96) 49.6 -> 43.7.
 // SK and BK give the split-K chunk as in kernels.py:271-272, kept a multiple of 64 (one
 // MFMA K step). GM and mma are accepted and do not change the schedule: INT8 MFMA gives the
 // bits of both of the reference's tensor-core paths.
@@ -219,8 +222,12 @@ int make_plan(int64_t K, const int32_t* cfg, int cfg_len, ExactPlan* out) {
     p.family = kFamilySmall;
     p.mt = BM <= 16 ? 1 : (BM <= 32 ? 2 : 4);
     p.nt = BN <= 16 ? 1 : (BN <= 32 ? 2 : 4);
-    if (BM <= 16 && (BN == 48 || BN == 80 || BN == 96) && warps == 8 && stages == 1) p.wide = BN / 16;
     int nwk = warps <= 4 ? 4 : (warps <= 8 ? 8 : 16);
+    if (BM <= 16 && (BN == 48 || BN == 80 || BN == 96) && warps == 8 && stages == 1) {
+      p.wide = BN / 16;
+      p.nt = p.wide == 3 ? 1 : 2;
+      nwk = 4;
+    }
     int chunk = stages <= 1 ? 1 : (stages <= 3 ? 2 : 4);
     bool found = false;
     for (int c = chunk; c >= 1 && !found; c >>= 1)
