@@ -49,11 +49,15 @@ def test_pack_matches_layout_and_digitize_packed(R, Kd):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("R,Kd", [(4096, 3072), (6500, 2040), (4100, 4097), (4111, 8136), (4097, 12288), (4100, 12296)])
+@pytest.mark.parametrize("R,Kd", [(4096, 3072), (6500, 2040), (4100, 4097), (4111, 8136), (4097, 12288), (4100, 12296),
+                                  (8225, 2040), (22000, 768), (6200, 3080), (4096, 4096), (4096, 4104), (7000, 8136),
+                                  (11281, 6152), (8190, 12280)])
 def test_digitize_packed_of_many_rows(dtype, R, Kd):
-    """Many rows are digitized a 16-row tile per workgroup (4, 8 or 12 steps a wave; rows that are not
-    16-byte aligned and longer rows keep a workgroup per row): the digits, sums and shifts of the
-    row-major kernel, packed, and the oracle's on the first and last rows; zero digits in the padding."""
+    """Many rows are digitized a 16-row tile per workgroup (the last eight sizes: 4, 8 or 12 steps a
+    wave, up to the edges of rows and columns) where that is faster; the sizes before them (few values,
+    nearly empty last rounds, rows that are not 16-byte aligned, longer rows) and F = 15 past 8192
+    columns keep a workgroup per row: the digits, sums and shifts of the row-major kernel, packed, and
+    the oracle's on the first and last rows; zero digits in the padding."""
     g = torch.Generator(device=DEV).manual_seed(R)
     x = torch.randn(R, Kd, device=DEV, generator=g) * 10 ** (torch.rand(R, 1, device=DEV, generator=g) * 6 - 3)
     x[5] = 0

@@ -294,16 +294,37 @@ __global__ __launch_bounds__(64 * NW) void digitize_tile_kernel(const uint16_t* 
   }
 }
 
+// Whether R packed rows take a workgroup per 16-row tile. Lines measured over 4096 to 32768 rows of
+// 512 to 12288 columns, F = 14 bf16 and F = 15 fp16, as the time of a workgroup per row over this:
+//  * at least 16 Mi values and 768 columns: below, 0.78-1.0 (10240 x 1536 0.95, 32768 x 512 0.85);
+//    from there 1.0-1.5 up to 2048 columns, whose workgroups run several to a CU;
+//  * up to 4096 columns, two or three workgroups to a CU: 0.8-1.0 at 257 to 383 tiles, where most
+//    CUs wait for the few with a second one, otherwise 0.98-1.4 (4096 x 4096 1.20, 24576 x 4096 1.12);
+//  * past 4096 columns one workgroup of 16 waves fills a CU, so a last round that is partly empty costs
+//    a whole one (4352 x 12288 0.78, 8704 x 6144 0.86): only where the rounds are 0.85 full (0.9 past two,
+//    with at least 6 of the 8 or 12 steps of a wave in use), 1.0-1.41; past four rounds 0.95-1.08;
+//  * F = 15 past 8192 columns would spill (12 steps and the digit sum in 128 VGPRs): 0.64-1.0 in fp16.
+bool tile_pays(int64_t R, int64_t K, int F) {
+  const int64_t KT = cdiv<int64_t>(K, 64), tiles = cdiv<int64_t>(R, 16), rounds = cdiv<int64_t>(tiles, 256);
+  if (R < 4096 || KT < 12 || KT > 192 || R * K < (int64_t)16 << 20) return false;
+  if (KT <= 32) return true;
+  if (KT <= 64) return tiles <= 256 || tiles >= 384;
+  if ((F == 15 && KT > 128) || rounds > 4 || (rounds > 2 && KT < 96)) return false;
+  return tiles * 20 >= rounds * 256 * (rounds <= 2 ? 17 : 18);
+}
+
 template <int DT, int NW, int XS>
 hipError_t launch_tile(const void* x, int64_t R, int64_t K, int64_t ldx, int8_t* out, int32_t* cs, int32_t* sh, int F,
                        hipStream_t st) {
   const dim3 grid((unsigned)cdiv<int64_t>(R, 16)), block(64 * NW);
   const uint16_t* xp = reinterpret_cast<const uint16_t*>(x);
   const int KT = (int)cdiv<int64_t>(K, 64);
-  if (F == 15)
+  if (F != 15)
+    hipLaunchKernelGGL((digitize_tile_kernel<DT, NW, XS, false>), grid, block, 0, st, xp, R, K, ldx, out, KT, cs, sh, F);
+  else if constexpr (XS <= 8)
     hipLaunchKernelGGL((digitize_tile_kernel<DT, NW, XS, true>), grid, block, 0, st, xp, R, K, ldx, out, KT, cs, sh, F);
   else
-    hipLaunchKernelGGL((digitize_tile_kernel<DT, NW, XS, false>), grid, block, 0, st, xp, R, K, ldx, out, KT, cs, sh, F);
+    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
@@ -360,11 +381,7 @@ hipError_t launch_digitize_fast(const void* x, int x_dtype, int64_t R, int64_t K
   const int cpt = digitize_fast_shape(K, &nthr);
   if (cpt == 0) return hipErrorInvalidValue;
   const int64_t KT = cdiv<int64_t>(K, 64);
-  // A workgroup per 16-row tile from one tile per CU on (4096 rows), and enough columns: measured,
-  // us, a workgroup per row / per tile: 2048 x 4096 11.4 / 12.5, 4096 x 4096 19.2 / 15.1, 24576 x
-  // 4096 90.1 / 79.4, 4096 x 12288 47.8 / 39.9, 8192 x 1024 10.5 / 11.1, 24576 x 1024 29.4 / 21.6.
-  if (packed && vec && x_dtype != VXA_F32 && R >= 4096 && R * K >= (int64_t)12 << 20 &&
-      cdiv<int64_t>(R, 16) <= 0x7FFFFFFFLL) {
+  if (packed && vec && x_dtype != VXA_F32 && tile_pays(R, K, F) && cdiv<int64_t>(R, 16) <= 0x7FFFFFFFLL) {
     const hipError_t err = x_dtype == VXA_BF16 ? dispatch_tile<VXA_BF16>(x, R, K, ldx, h, cs, sh, F, st)
                                                : dispatch_tile<VXA_F16>(x, R, K, ldx, h, cs, sh, F, st);
     if (err != hipErrorInvalidValue) return err;
