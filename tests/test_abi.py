@@ -90,6 +90,25 @@ def test_paged_workspace_sizes():
     assert nx.paged_workspace(4, 16, 256, 9000, 4096) == 4 * 16 * 3 * 258 * 4
 
 
+def test_units_workspace_is_bounded():
+    """The partials of every 64-key unit where a small grid computes its units apart, otherwise the
+    segments' partials: not where a segment is much longer than the keys or the partials are large."""
+    def units(n, H, KV, D, keys, split=2048, blk=16, waves=4):
+        return nx.paged_units_workspace(n, H, KV, D, keys, split, blk, waves)
+
+    assert units(1, 32, 8, 128, 16384) == 32 * 8 * 32 * 130 * 4
+    assert units(2, 32, 8, 128, 16384) == 2 * units(1, 32, 8, 128, 16384)
+    assert units(4, 32, 8, 128, 16384) == nx.paged_workspace(4, 32, 128, 16384, 2048)  # more than 128 segments
+    assert units(16, 32, 8, 128, 600) == 16 * 32 * 32 * 130 * 4
+    assert units(16, 32, 8, 128, 256) == 0 and units(16, 32, 32, 64, 512) == 0  # few keys
+    assert units(16, 32, 8, 128, 600, blk=32) == 0 and units(16, 32, 8, 128, 600, waves=8) == 0
+    # one segment of 131040 keys: 16 units are needed at a bound of 1000 keys, 2048 would be held
+    assert units(16, 32, 8, 128, 1000, split=131040) == 0
+    assert units(1, 8, 1, 64, 1000, split=131040) == 0
+    assert units(1, 8, 1, 64, 131040, split=131040) == 8 * 2048 * 66 * 4
+    assert units(64, 16, 2, 256, 131040, split=131040) == 0  # 2 GB of partials
+
+
 def test_entry_points_validate_before_launching():
     L = nx.lib()
     # digitize: F outside 1..15 and negative sizes are argument errors; zero rows is a no-op

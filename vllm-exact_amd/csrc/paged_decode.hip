@@ -739,6 +739,10 @@ int64_t num_segments(int64_t max_len, int64_t split) {
 
 int64_t units_of(int64_t split) { return cdiv<int64_t>(split, kUnit); }
 
+size_t units_bytes(int64_t n, int64_t num_heads, int64_t head_dim, int64_t ns, int64_t split) {
+  return (size_t)n * num_heads * ns * units_of(split) * (head_dim + 2) * sizeof(float);
+}
+
 // Whether the units of a grid of ns segments per request are computed apart. keys is the most
 // keys a request of the grid may have. Measured at H32/KV8/D128 (us a call, whole segments /
 // units): 1 request of 520 keys 13.1 / 10.9, 1024 18.5 / 11.2, 16384 35.3 / 21.2 (64 workgroups of
@@ -748,14 +752,15 @@ int64_t units_of(int64_t split) { return cdiv<int64_t>(split, kUnit); }
 // costs what the shorter chains gain, unless a key is much work (G query heads of D dims): 1 request
 // of 400 keys 8.9 / 9.1 at G = 4, D = 64, 11.7 / 10.8 at D = 128, 20.7 / 14.3 at D = 256, 9.1 / 9.5 at
 // G = 1, D = 128, 17.6 / 13.1 at D = 256, 27.8 / 18.3 at G = 8, D = 256.
-bool use_units(int64_t n, int64_t num_heads, int64_t kv_heads, int64_t head_dim, int64_t ns, int64_t keys, int64_t blk,
-               int64_t waves) {
+// The grid and the workspace hold every unit of a segment (a request past the caller's bound but inside
+// its segment is computed too), so a segment much longer than the keys (more than 8 times their units)
+// or partials past 256 MiB keep whole segments: 16 requests bounded by 1000 keys in segments of 131040
+// would take 545 MB and 512 workgroups a head, 4 of them with keys. Segments of 2048 never do.
+bool use_units(int64_t n, int64_t num_heads, int64_t kv_heads, int64_t head_dim, int64_t ns, int64_t split, int64_t keys,
+               int64_t blk, int64_t waves) {
   const bool much = head_dim >= 256 || num_heads / kv_heads * head_dim >= 512;
-  return blk == 16 && waves == 4 && keys > (much ? 4 : 8) * kUnit && n * kv_heads * ns <= 128;
-}
-
-size_t units_bytes(int64_t n, int64_t num_heads, int64_t head_dim, int64_t ns, int64_t split) {
-  return (size_t)n * num_heads * ns * units_of(split) * (head_dim + 2) * sizeof(float);
+  if (blk != 16 || waves != 4 || keys <= (much ? 4 : 8) * kUnit || n * kv_heads * ns > 128) return false;
+  return units_of(split) <= 8 * units_of(keys) && units_bytes(n, num_heads, head_dim, ns, split) <= (size_t)256 << 20;
 }
 
 }  // namespace
@@ -767,7 +772,8 @@ extern "C" int vxa_paged_decode_units_workspace(int64_t n, int64_t num_heads, in
   if (rc != VXA_OK) return rc;
   if (num_kv_heads <= 0 || blk <= 0 || waves <= 0) return VXA_ERR_ARG;
   const int64_t ns = num_segments(max_len, split);
-  if (use_units(n, num_heads, num_kv_heads, head_dim, ns, max_len, blk, waves)) *ws_bytes = units_bytes(n, num_heads, head_dim, ns, split);
+  if (use_units(n, num_heads, num_kv_heads, head_dim, ns, split, max_len, blk, waves))
+    *ws_bytes = units_bytes(n, num_heads, head_dim, ns, split);
   return VXA_OK;
 }
 
@@ -841,7 +847,7 @@ int paged_decode_impl(const void* q, int64_t sqt, int64_t sqh, const void* k_cac
   pp.n_live = n_live;
   PagedMode mode = kSegments;
   const int64_t keys = max_seq_len > 0 ? std::min(max_len, max_seq_len) : max_len;
-  if (use_units(n, num_heads, num_kv_heads, head_dim, ns, keys, blk, waves) && ws &&
+  if (use_units(n, num_heads, num_kv_heads, head_dim, ns, split, keys, blk, waves) && ws &&
       ws_bytes >= units_bytes(n, num_heads, head_dim, ns, split))
     mode = kUnits;
   pp.units = (int32_t)units_of(split);
