@@ -333,3 +333,20 @@ def test_keys_that_score_minus_infinity_weigh_nothing(monkeypatch, BS, blk, wave
     monkeypatch.setattr(P._nx, "paged_units_workspace", lambda n, H, KV, *a: P._nx.paged_workspace(n, H, *a[:-2]))
     assert torch.equal(_run(*gpu, 0.09, B, D, blk=blk, warps=waves, split=split).view(torch.int32), whole.view(torch.int32))
     _check_tol(whole.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("G", [4, 8])
+def test_other_constant_sets_of_wide_heads(G):
+    """32 keys a step on 8 waves, 256 dims: a wave's whole share runs as one unit at 8 heads a group
+    (the registers hold no second state), 64 keys at a time at 4. Lengths around a step, the waves'
+    first steps and a segment, against the float64 oracle, the same bits alone as in the batch."""
+    D, KV, split = 256, 2, 528
+    lens = [1, 31, 33, 256, 257, 527, 528, 529, 1300]
+    q, kv, bt, sl = make_paged(len(lens), 1300, 16, G * KV, KV, D, seed=G)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    q, kv, bt, sl = (t.to(DEV) for t in (q, kv, bt, sl))
+    full = _run(q, kv, bt, sl, 1 / 16, len(lens), D, blk=32, warps=8, split=split)
+    for b in (2, 7, 8):
+        alone = _run(q[b:b + 1], kv, bt[b:b + 1], sl[b:b + 1], 1 / 16, 1, D, blk=32, warps=8, split=split)
+        assert torch.equal(alone[0], full[b]), lens[b]
+    _check_tol(full.cpu().numpy(), _oracle(q, kv, bt, sl, 1 / 16, len(lens), D))

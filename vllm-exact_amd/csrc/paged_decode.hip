@@ -204,6 +204,11 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   constexpr int DPL = DimTraits<D>::kDpl;
   constexpr int FL = G * DPL;  // accumulators of a lane
   constexpr int QF = FL / 4;   // and the quarter of them its row owns once the rows are summed
+  // 8 waves of 128 accumulators a lane and two tiles a step (8 heads of 256 dims at 32 keys) have no
+  // registers for a running state beside a unit's: there a wave's whole share is one unit. 64 requests
+  // of 2048 to 4096 keys, us: 278 before there were units, 367 with a merge per 64 keys (113 VGPRs
+  // spilled), 290 this way.
+  constexpr bool ONE_UNIT = !AHEAD && FL >= 128 && TPG == 2 && NW == 8;
   __shared__ float s_m[NW][G];
   __shared__ float s_l[NW][G];
   __shared__ float s_acc[NW][G][D];
@@ -337,7 +342,7 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   // One unit of this wave; `next` (AHEAD): the wave has a further unit, NW units on.
   auto unit = [&](int u, auto next) {
     const int ubase = start + u * kUnit;
-    const int uend = min(ubase + kUnit, end);
+    const int uend = ONE_UNIT ? end : min(ubase + kUnit, end);
     float m_run = kNegInf, l_run = 0.0f;  // per head column (S layout)
     float acc[FL];                         // PV layout: head x owned dims
 #pragma unroll
@@ -423,7 +428,8 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
         }
       }
     } else {
-      for (int kbase = ubase; kbase < uend; kbase += 16 * TPG) {
+      constexpr int kStep = 16 * TPG;
+      for (int kbase = ONE_UNIT ? start + wave * kStep : ubase; kbase < uend; kbase += ONE_UNIT ? NW * kStep : kStep) {
         const uint16_t* krow[TPG];
 #pragma unroll
         for (int t = 0; t < TPG; ++t) krow[t] = krow_of(kbase + 16 * t);
@@ -458,6 +464,11 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
         const int f = row * QF + i;
         p.ap[(((int64_t)b * p.H + g * G + f / DPL) * nu + ui) * D + col * DPL + f % DPL] = acc[i];
       }
+    } else if constexpr (ONE_UNIT) {
+      m_tot = m_run;
+      l_tot = l_run;
+#pragma unroll
+      for (int i = 0; i < QF; ++i) a_tot[i] = acc[i];
     } else {
       // merge_state of the running state with the unit's, the factors computed once per head
       const float mn = fmaxf(m_tot, m_run);
@@ -483,6 +494,8 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
       for (; u + NW < nunit; u += NW) unit(u, std::true_type{});
       unit(u, std::false_type{});
     }
+  } else if constexpr (ONE_UNIT) {
+    unit(0, std::false_type{});
   } else {
     for (int u = wave; u < nunit; u += NW) unit(u, std::false_type{});
   }
