@@ -77,6 +77,10 @@ struct PagedParams {
 };
 
 constexpr float kNegInf = -__builtin_huge_valf();
+// Where a unit's running maximum starts: below every finite score, so that the first tile replaces it,
+// and finite, so that keys scoring -inf weigh exp2(-inf - m) = 0 also where nothing else has been seen
+// (-inf - -inf would be NaN). Such a unit's state is (kLowest, 0, 0), which adds 0 to any merge.
+constexpr float kLowest = -3.402823466e38f;  // -FLT_MAX
 
 __device__ inline float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -343,7 +347,7 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
   auto unit = [&](int u, auto next) {
     const int ubase = start + u * kUnit;
     const int uend = ONE_UNIT ? end : min(ubase + kUnit, end);
-    float m_run = kNegInf, l_run = 0.0f;  // per head column (S layout)
+    float m_run = kLowest, l_run = 0.0f;  // per head column (S layout)
     float acc[FL];                         // PV layout: head x owned dims
 #pragma unroll
     for (int i = 0; i < FL; ++i) acc[i] = 0.0f;
@@ -371,16 +375,13 @@ __global__ __launch_bounds__(64 * NW) void paged_partial_kernel(PagedParams p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[t][r]);
       const float m_new = fmaxf(m_run, rows_max(mx));
-      // Where every score so far is -inf (m_new too), the differences are taken to 0: the keys weigh 0
-      // and the state stays (-inf, 0, 0), which a later merge drops; -inf - -inf would be NaN.
-      const float m_ref = (m_new == kNegInf) ? 0.0f : m_new;
-      const float alpha = exp2_hw(m_run - m_ref);  // m_run == -inf -> 0
+      const float alpha = exp2_hw(m_run - m_new);  // m_run == kLowest -> 0, or nothing to rescale
       float psum = 0.0f;
 #pragma unroll
       for (int t = 0; t < TPG; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          sc[t][r] = exp2_hw(sc[t][r] - m_ref);
+          sc[t][r] = exp2_hw(sc[t][r] - m_new);
           psum += sc[t][r];
         }
       l_run = fmaf(l_run, alpha, rows_sum(psum));
