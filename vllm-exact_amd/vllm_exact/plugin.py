@@ -188,22 +188,23 @@ def _(x, wh, wl, cw, sw):
     return x.new_empty(*x.shape[:-1], sw.shape[0])
 
 
-# (M, N, K, dtype, F, TRUNC, aligned bf16 rows) -> how the op runs such a packed call: (packed weight
-# shape, one launch, cfg array, its length, n1, cfg2 array, its length, scratch bytes). Sizes and
-# alignment only; cleared by load_table, and when it holds MAX_PLANS (row counts vary without bound
-# under a server).
+# (M, N, K, dtype, F, TRUNC) -> how the op runs such a packed call: (packed weight shape, one launch,
+# cfg array, its length, n1, cfg2 array, its length, scratch bytes); with a seventh item, False, the
+# plan of rows that are not 16-byte aligned, where the first is for one launch. Sizes and alignment
+# only; cleared by load_table, and when it holds MAX_PLANS (row counts vary without bound under a
+# server).
 _PLANS = {}
 MAX_PLANS = 4096
 
 
-def _op_plan(M, N, Kd, dtype, aligned):
+def _op_plan(M, N, Kd, dtype, aligned=True):
     cfg, one_launch = _packed_plan(M, N, Kd, dtype, aligned)
     n1, cfg2 = _n_split(M, N, Kd) or (0, None)
     arr, n, arr2, n2, scratch = _nx.op_scratch(M, N, Kd, cfg, n1, cfg2)
     if len(_PLANS) >= MAX_PLANS:
         _PLANS.clear()
     plan = (torch.Size(K.packed_shape(N, Kd)), one_launch, arr, n, n1, arr2, n2, scratch)
-    _PLANS[(M, N, Kd, dtype, F, TRUNC, aligned)] = plan
+    _PLANS[(M, N, Kd, dtype, F, TRUNC) + (() if aligned else (False,))] = plan
     return plan
 
 
@@ -230,8 +231,9 @@ def _linear_cuda(x, wh, wl, cw, sw):
             # a one-row tensor may have any row stride: it is never used
             ldx = x2.stride(0) if M > 1 else max(x2.stride(0), Kd)
             xptr = x2.data_ptr()
-            aligned = dtype == torch.bfloat16 and xptr % 16 == 0 and ldx % 8 == 0
-            plan = _PLANS.get((M, N, Kd, dtype, F, TRUNC, aligned)) or _op_plan(M, N, Kd, dtype, aligned)
+            plan = _PLANS.get((M, N, Kd, dtype, F, TRUNC)) or _op_plan(M, N, Kd, dtype)
+            if plan[1] and (xptr % 16 or ldx % 8):
+                plan = _PLANS.get((M, N, Kd, dtype, F, TRUNC, False)) or _op_plan(M, N, Kd, dtype, False)
             shape, one_launch, arr, n, n1, arr2, n2, scratch = plan
             if wh.shape == shape:
                 out = x2.new_empty(M, N)
@@ -249,8 +251,7 @@ def _linear_cuda(x, wh, wl, cw, sw):
                 if status == _nx.VXA_OK:
                     return out if len(shp) == 2 else out.reshape(*shp[:-1], N)
                 if one_launch and status == _nx.VXA_ERR_UNSUPPORTED:
-                    # planned anew once the general body knows why
-                    _PLANS.pop((M, N, Kd, dtype, F, TRUNC, aligned), None)
+                    _PLANS.pop((M, N, Kd, dtype, F, TRUNC), None)  # planned anew once the general body knows why
                 else:
                     _nx.check(status, "exactmm::linear")
     return _linear_body(x, wh, wl, cw, sw)
