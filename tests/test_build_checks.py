@@ -1,10 +1,15 @@
 """CPU tests of the build-time assembly check for inline-asm loads
 (vllm-exact_amd/check_async_loads.py): it must reject a destination register touched before
 the covering wait (straight line, through a branch, around a loop), a path that ends
-uncovered, and compiler-generated M0 use, and accept the same code once a wait covers it."""
+uncovered, and compiler-generated M0 use, and accept the same code once a wait covers it; and of
+the registers of the built kernels."""
+import re
+import struct
 import subprocess
 import sys
 from pathlib import Path
+
+import msgpack
 
 ROOT = Path(__file__).resolve().parents[1]
 CHECK = ROOT / "vllm-exact_amd" / "check_async_loads.py"
@@ -52,3 +57,30 @@ def test_rejects_uncovered_end_and_loop_reuse(tmp_path):
 def test_rejects_compiler_m0_use(tmp_path):
     r = run(tmp_path, "s_mov_b32 m0, s2\n" + LOAD + "s_waitcnt vmcnt(0)\ns_endpgm")
     assert r.returncode == 1 and "m0" in r.stdout
+
+
+def kernel_metadata(lib):
+    """The kernels' metadata (AMDGPU notes, msgpack) of every gfx950 code object in the library."""
+    data, pos = lib.read_bytes(), 0
+    while (pos := data.find(b"\x7fELF", pos)) >= 0:
+        if struct.unpack_from("<H", data, pos + 18)[0] == 224:  # e_machine: EM_AMDGPU
+            shoff, = struct.unpack_from("<Q", data, pos + 40)
+            shentsize, shnum = struct.unpack_from("<HH", data, pos + 58)
+            for i in range(shnum):
+                _, kind, _, _, offset = struct.unpack_from("<IIQQQ", data, pos + shoff + i * shentsize)
+                if kind == 7:  # SHT_NOTE: sizes of the name and of the contents, type, name padded to 4
+                    name, size, _ = struct.unpack_from("<III", data, pos + offset)
+                    at = pos + offset + 12 + (name + 3) // 4 * 4
+                    yield from msgpack.unpackb(data[at:at + size]).get("amdhsa.kernels", [])
+        pos += 4
+
+
+def test_kernels_use_no_scratch():
+    """No kernel spills, but paged decode away from the default constants (16 keys a step, 4 waves):
+    its steps of 64 keys or 8 waves of many heads have more accumulators than registers."""
+    kernels = list(kernel_metadata(ROOT / "vllm-exact_amd" / "vllm_exact" / "libvllm_exact_amd.so"))
+    assert len(kernels) > 100
+    for k in kernels:
+        paged = re.search(r"paged_partial_kernelILi\d+ELi\d+ELi(\d+)ELi(\d+)E", k[".name"])
+        if not paged or paged.groups() == ("1", "4"):
+            assert k[".private_segment_fixed_size"] == 0, k[".name"]

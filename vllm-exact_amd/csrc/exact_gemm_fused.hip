@@ -501,7 +501,9 @@ __global__ __launch_bounds__(64 * NWK) void exact_fused_xreg_kernel(FusedParams 
   if constexpr (OFFSET) {
     cs += __shfl_xor(cs, 16);
     cs += __shfl_xor(cs, 32);
-    if (kq == 0) s_cs[wave][r16] = cs;
+    int t = threadIdx.x;  // the row from here on anew: its LDS offset held over the K loop spills at 6 tiles
+    asm volatile("" : "+v"(t));
+    if (kq == 0) s_cs[wave][t & 15] = cs;
   }
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
