@@ -107,6 +107,9 @@ def test_units_workspace_is_bounded():
     assert units(1, 8, 1, 64, 1000, split=131040) == 0
     assert units(1, 8, 1, 64, 131040, split=131040) == 8 * 2048 * 66 * 4
     assert units(64, 16, 2, 256, 131040, split=131040) == 0  # 2 GB of partials
+    for bad in (dict(KV=0), dict(n=-1), dict(H=0), dict(D=0), dict(split=0), dict(blk=0), dict(waves=0)):
+        with pytest.raises(ValueError):
+            units(**dict(dict(n=1, H=32, KV=8, D=128, keys=16384), **bad))
 
 
 def test_entry_points_validate_before_launching():
@@ -186,6 +189,49 @@ def test_fused_entry_point_validates_before_launching():
     assert call(ldx=100) == nx.VXA_ERR_ARG
     assert call(x=None) == nx.VXA_ERR_ARG
     assert call(w=fake + 8) == nx.VXA_ERR_ARG
+
+
+def test_op_scratch_sizes_and_arguments():
+    """vxa_exact_linear_op_scratch: the packed digits, sums and shifts of x, each rounded up to 256
+    bytes, and the larger split-K workspace of the one or two GEMMs."""
+    L = nx.lib()
+    one, split, other = (nx.cfg_array(c) for c in ((16, 64, 128, 4, 3, 8, 1), (64, 64, 128, 4, 3, 8, 4), (64, 64, 128, 4, 3, 8, 2)))
+
+    def call(m=100, n=512, k=1000, cfg=one, n1=0, cfg2=(None, 0)):
+        out = ctypes.c_size_t(7)
+        return L.vxa_exact_linear_op_scratch(m, n, k, *cfg, n1, *cfg2, ctypes.byref(out)), out.value
+
+    digits = 7 * 16 * 2048 + 2 * 512
+    assert call() == (nx.VXA_OK, digits)
+    assert call(cfg=split) == (nx.VXA_OK, digits + 4 * 100 * 512 * 8)
+    assert call(cfg=split, n1=64, cfg2=other) == (nx.VXA_OK, digits + 2 * 100 * 448 * 8)
+    assert call(cfg=split, n1=512, cfg2=other) == (nx.VXA_OK, digits + 4 * 100 * 512 * 8)
+    assert call(m=0) == (nx.VXA_OK, 0)
+    for bad in (dict(m=-1), dict(n=-1), dict(k=-1), dict(n1=-16, cfg2=one), dict(n1=24, cfg2=one), dict(n1=528, cfg2=one),
+                dict(n1=64), dict(n1=64, cfg2=nx.cfg_array((0, 64, 128, 4, 3, 8))), dict(cfg=(None, 0))):
+        assert call(**bad)[0] == nx.VXA_ERR_ARG, bad
+    assert L.vxa_exact_linear_op_scratch(1, 1, 1, *one, 0, None, 0, None) == nx.VXA_ERR_ARG
+
+
+def test_op_entry_validates_before_launching():
+    """vxa_exact_linear_op: what is refused is refused before the digitize launch (the pointers are
+    never dereferenced and no GPU is needed)."""
+    L = nx.lib()
+    fake = 0x1000
+    cfg = nx.cfg_array((16, 64, 128, 4, 1, 8, 1))
+
+    def call(x=fake, xd=nx.VXA_BF16, ldx=64, wp=fake, cw=fake, sw=fake, out=fake, od=nx.VXA_BF16, ldo=64, m=2, n=64,
+             k=64, f=14, trunc=1, cfg=cfg, n1=0, cfg2=(None, 0), scratch=fake, size=1 << 20):
+        return L.vxa_exact_linear_op(x, xd, ldx, wp, cw, sw, out, od, ldo, m, n, k, f, trunc, *cfg, n1, *cfg2, scratch,
+                                     size, None)
+
+    for bad in (dict(x=None), dict(xd=7), dict(ldx=10), dict(wp=None), dict(wp=fake + 8), dict(sw=None), dict(out=None),
+                dict(od=9), dict(ldo=10), dict(f=15, trunc=0, cw=None), dict(f=0), dict(f=16), dict(m=-1), dict(n1=8, cfg2=cfg),
+                dict(n1=80, cfg2=cfg), dict(n1=16), dict(cfg=(None, 0)), dict(scratch=fake + 16)):
+        assert call(**bad) == nx.VXA_ERR_ARG, bad
+    need = 2048 + 2 * 256
+    assert call(size=need - 1) == nx.VXA_ERR_WORKSPACE and call(scratch=None) == nx.VXA_ERR_WORKSPACE
+    assert call(m=0) == nx.VXA_OK and call(n=0, n1=0) == nx.VXA_OK
 
 
 def test_noalloc_entry_refuses_problems_beyond_its_scratch():

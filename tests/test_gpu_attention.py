@@ -78,11 +78,13 @@ def test_device_count_limits_the_requests(L):
         P.paged_decode(q, kc, vc, bt, sl, scale, out, B, 0, n_live=torch.tensor([1], device=DEV))
 
 
+@pytest.mark.parametrize("units", [True, False])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
-def test_length_bound_trims_the_grid_without_changing_bits(out_dtype):
+def test_length_bound_trims_the_grid_without_changing_bits(monkeypatch, out_dtype, units):
     """max_seq_len as a bound on the batch's lengths (0: none, the grid of MAX_LEN): the grid
-    then covers only the segments the bound reaches, 3 of the 8 at 5000 keys and 1 at 2048 (no
-    merge launch). Requests within the bound keep the full grid's bits, single- and
+    then covers only the segments the bound reaches, 3 of the 8 at 5000 keys and 1 at 2048. These
+    grids take units in workgroups of their own where the workspace holds their partials, and whole
+    segments otherwise (a bound of one segment then has no merge launch). Requests within the bound keep the full grid's bits, single- and
     multi-segment alike; a request longer than the bound gets NaN rows and leaves the others
     unchanged. The same through the device-count entry point."""
     B, H, KV, D = 6, 8, 2, 128
@@ -92,6 +94,8 @@ def test_length_bound_trims_the_grid_without_changing_bits(out_dtype):
     kc, vc = kv_views(kv, D)
     scale = D ** -0.5
     assert P.MAX_LEN == 16384 and P.SPLIT == 2048
+    if not units:
+        monkeypatch.setattr(P._nx, "paged_units_workspace", lambda n, H, KV, *a: P._nx.paged_workspace(n, H, *a[:-2]))
 
     def run(bound, n_live=None):
         out = torch.full((B, H, D), float("nan"), device=DEV, dtype=out_dtype)

@@ -58,7 +58,7 @@ constexpr Candidate kThreeDots[] = {
     {true, 64, 16, 32, 128, 16, 1, 0.833f, 2.820f, 2.003f, 0.052f, 0.000f, 0.000f},
     {true, 4, 16, 64, 128, 8, 1, 0.000f, 3.714f, 2.001f, 0.095f, 0.000f, 0.000f},
     {true, 64, 16, 64, 128, 8, 1, 1.345f, 2.256f, 2.989f, 0.080f, 0.000f, 0.000f},
-{true, 4, 16, 48, 128, 8, 1, 2.955f, 0.000f, 1.563f, 0.098f, 0.000f, 0.000f},
+    {true, 4, 16, 48, 128, 8, 1, 2.955f, 0.000f, 1.563f, 0.098f, 0.000f, 0.000f},
     {true, 64, 16, 48, 128, 8, 1, 3.128f, 0.000f, 1.981f, 0.091f, 0.000f, 0.000f},
     {true, 4, 16, 80, 128, 8, 1, 0.906f, 2.809f, 2.485f, 0.083f, 0.000f, 0.000f},
     {true, 64, 16, 80, 128, 8, 1, 0.700f, 3.839f, 2.744f, 0.080f, 0.000f, 0.000f},

@@ -8,8 +8,8 @@
 // other requests, or on where the pages sit in memory.
 //
 // Kernel shape (MI355X-first, not a translation of the Triton kernel):
-//  * a segment is cut into units of 64 keys; a wave runs an online softmax over one unit at a
-//    time and merges its units (wave, wave + NW, ...) in order, the NW waves of the segment are
+//  * a segment is cut into units of 64 keys (one exception: ONE_UNIT); a wave runs an online softmax
+//    over one unit at a time and merges its units (wave, wave + NW, ...) in order, the NW waves of the segment are
 //    merged in order, then the segments. A workgroup computes a whole segment of (request b, KV
 //    head g); where that leaves most CUs idle (a few requests), it computes NW units only and
 //    writes their partials, which a second kernel merges in the same order: the same bits;
@@ -188,8 +188,13 @@ __device__ inline VRaw<D> load_v(const uint16_t* p) {
   return r;
 }
 
-// Tiles of 16 keys whose K and V loads a wave has in flight when AHEAD: 128 VGPRs of them (64
-// where the accumulators of 4 or 8 heads of 256 dims need the registers: two waves a SIMD at 4).
+// Tiles of 16 keys whose K and V loads a wave has in flight when AHEAD: at D = 128 four tiles, 128
+// VGPRs and 32 KiB; at D = 256 two, the same, or one (64 VGPRs) where the accumulators of 4 or 8 heads
+// need the registers (4 heads keep two waves a SIMD); at D = 64 four, 64 VGPRs and 16 KiB (a ring
+// is at most a unit's tiles). 8 heads of 128 dims on whole segments (260 VGPRs) and 2 of 256 (260-268)
+// leave one wave a SIMD and are still faster than without the ring at more waves: 64 requests of
+// 4096 to 8192 keys, 4 KV heads, D = 128, G = 8 220.8 -> 183.6 us, 256 of 512 to 1024 109.2 -> 102.2;
+// 8 KV heads, D = 256, G = 2, 64 of 1024 to 2048 170.1 -> 163.7, 256 of 512 to 1024 325.1 -> 308.8.
 template <int D, int G>
 constexpr int ahead_tiles() {
   return D == 256 ? (G >= 4 ? 1 : 2) : 4;
@@ -634,7 +639,7 @@ __global__ __launch_bounds__(1024) void paged_merge_units_kernel(PagedParams p) 
 
 template <int D>
 void launch_merge_units(const PagedParams& pp, int64_t heads, hipStream_t st) {
-  if (D > 32 && heads * (D / 32) <= 256)
+  if (heads * (D / 32) <= 256)
     hipLaunchKernelGGL((paged_merge_units_kernel<D, 4, true>), dim3((unsigned)(heads * (D / 32))), dim3(1024), 0, st, pp);
   else
     hipLaunchKernelGGL((paged_merge_units_kernel<D, 4, false>), dim3((unsigned)heads), dim3(1024), 0, st, pp);
