@@ -97,7 +97,7 @@ int vxa_exact_linear(const int8_t* xh, const int8_t* xl, const int32_t* cx, cons
  * The config of a packed exact linear of [m, k] x [n, k] where no tuning table names one: the
  * candidate with the least time in a cost model of the kernels (host arithmetic only, no device
  * call). trunc as in vxa_exact_linear; one_launch_ok: the call may digitize inside the GEMM
- * launch (bf16 rows, vxa_exact_linear_bf16x). Writes a cfg of 7 entries and whether it is for
+ * launch (16-byte aligned bf16 rows, vxa_exact_linear_bf16x). Writes a cfg of 7 entries and whether it is for
  * vxa_exact_linear_bf16x (*one_launch = 1) or vxa_exact_linear_packed (0). Speed only.
  */
 int vxa_exact_linear_pick(int64_t m, int64_t n, int64_t k, int trunc, int one_launch_ok,
@@ -160,7 +160,9 @@ int vxa_exact_linear_bf16x(const void* x, int64_t ldx, const int8_t* wp, const i
  *         [n1, n) with cfg2
  *   scratch  256-byte aligned, at least the bytes of vxa_exact_linear_op_scratch with the same
  *         sizes and cfgs: the packed digits, their sums and shifts, and the split-K partials
- * Other arguments as vxa_digitize_packed and vxa_exact_linear_packed.
+ * Other arguments as vxa_digitize_packed and vxa_exact_linear_packed, checked before the first
+ * launch. A limit of the GEMM's own (VXA_ERR_UNSUPPORTED, a launch error) is reported after the
+ * digitize launch, which has written the scratch only.
  */
 int vxa_exact_linear_op_scratch(int64_t m, int64_t n, int64_t k, const int32_t* cfg, int cfg_len,
                                 int64_t n1, const int32_t* cfg2, int cfg2_len, size_t* bytes);
@@ -181,8 +183,9 @@ int vxa_paged_decode_workspace(int64_t n, int64_t num_heads, int64_t head_dim, i
 /*
  * Workspace bytes with which vxa_paged_decode also splits the segments of a small grid (few
  * requests) into units of 64 keys computed by workgroups of their own: the partials of every
- * unit where that applies, otherwise the bytes of vxa_paged_decode_workspace. blk and waves as
- * in vxa_paged_decode; max_len as in vxa_paged_decode_workspace. Either size is accepted, and
+ * unit where that applies, otherwise the bytes of vxa_paged_decode_workspace (also in segments
+ * much longer than max_len and past 256 MiB of partials). blk and waves as in vxa_paged_decode;
+ * max_len as in vxa_paged_decode_workspace. Either size is accepted, and
  * both give the same bits: the smaller one computes whole segments.
  */
 int vxa_paged_decode_units_workspace(int64_t n, int64_t num_heads, int64_t num_kv_heads,

@@ -602,14 +602,14 @@ hipError_t launch(const FusedParams& fp, hipStream_t st) {
 }
 
 // The wide x-in-registers tiles: NT = 3, 5 or 6 column tiles, 8 waves, K up to 4096 columns (8
-// steps a wave), any grid. They fill the CUs where 1, 2 or 4 tiles leave a last round nearly empty
+// steps a wave), any grid; at most 256 VGPRs and no scratch. They fill the CUs where 1, 2 or 4 tiles leave a last round nearly empty
 // or some CUs idle, and read x once per 48 to 96 columns, where the row pass reads it twice per 16
 // to 64 (a CU loads bytes from L2 at ~83 KB/us, which at 16 rows costs as much as the weights of 16
 // columns). Measured at K = 4096, us, best narrower tile -> wide: N = 10240 18.3 -> 17.0 at M = 1,
 // 20.0 -> 19.1 at 16 (F = 15: 22.0 -> 19.3); N = 20480 35.4 -> 32.3 at 16 (F = 15: 38.3 -> 32.7); N
 // = 24576 37.4 -> 37.7 at 16 (F = 15: 40.2 -> 38.4). At N = 8192 and 32768, whole rounds of the
-// narrower tiles, they lose (15.3 -> 17.0, 48.0 -> 52.3 at 16). hipErrorInvalidValue where a plan names none or K is longer: the small-M
-// kernel's tile of the plan then runs.
+// narrower tiles, they lose (15.3 -> 17.0, 48.0 -> 52.3 at 16). hipErrorInvalidValue where a plan
+// names none or K is longer: the small-M kernel's tile of the plan then runs.
 template <int NT, bool TRUNC>
 hipError_t launch_wide(const FusedParams& fp, hipStream_t st) {
   const int64_t blocks = cdiv<int64_t>(fp.M, 16) * cdiv<int64_t>(fp.N, 16 * NT);

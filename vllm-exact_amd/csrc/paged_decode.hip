@@ -9,10 +9,10 @@
 //
 // Kernel shape (MI355X-first, not a translation of the Triton kernel):
 //  * a segment is cut into units of 64 keys (one exception: ONE_UNIT); a wave runs an online softmax
-//    over one unit at a time and merges its units (wave, wave + NW, ...) in order, the NW waves of the segment are
-//    merged in order, then the segments. A workgroup computes a whole segment of (request b, KV
-//    head g); where that leaves most CUs idle (a few requests), it computes NW units only and
-//    writes their partials, which a second kernel merges in the same order: the same bits;
+//    over one unit at a time and merges its units (wave, wave + NW, ...) in order, the NW waves of
+//    the segment are merged in order, then the segments. A workgroup computes a whole segment of
+//    (request b, KV head g); where that leaves most CUs idle (a few requests), it computes NW units
+//    only and writes their partials, which a second kernel merges in the same order: the same bits;
 //  * S = K q^T on bf16 matrix cores (v_mfma_f32_16x16x32_bf16): rows are 16 keys of a tile,
 //    columns the G query heads of the group (bf16 x bf16 products are exact in fp32);
 //  * online softmax in base 2 on the hardware v_exp_f32, state per head kept in fp32;

@@ -199,8 +199,9 @@ def exact_linear_packed(xp, wp, K, F, trunc=False, out=None, cfg=None):
     return out
 
 
-# Without a tuning-table entry that says otherwise, the exactmm::linear op digitizes inside the
-# GEMM launch (exact_linear_bf16x) up to this many rows. Measured on MI355X the one launch
+# Where a shape's tuning-table row has no "one_launch" list, the exactmm::linear op digitizes inside
+# the GEMM launch (exact_linear_bf16x) up to this many rows (shapes without a row: the library's
+# choice by size). Measured on MI355X the one launch
 # saves 2-6 µs per op at 1-4 rows at every decode shape. Above that it depends on the shape:
 # every workgroup reads its x rows twice (row pass, then K loop), so at 16 rows it still wins
 # where K = 4096 and loses where K = 12288, and at 64 rows it loses. The tuner times both.

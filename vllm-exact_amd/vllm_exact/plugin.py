@@ -80,8 +80,8 @@ def _cfg(M, N, Kd):
 
 
 def _one_launch(M, N, Kd):
-    """Whether an (M, N, K) call takes the one-launch digitize + GEMM path: as the table row
-    that _cfg picks says when the shape's row has a "one_launch" list, else M <= 4
+    """Whether an (M, N, K) call of a shape in the table takes the one-launch digitize + GEMM path:
+    as the table row that _cfg picks says when the shape's row has a "one_launch" list, else M <= 4
     (K.ONE_LAUNCH_MAX_ROWS). Either way the bits are those of the two-launch path."""
     if _TABLE is not None and (N, Kd) in _ONE_LAUNCH_ROWS:
         ms = sorted(_TABLE[(N, Kd)])
